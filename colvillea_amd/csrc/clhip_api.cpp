@@ -160,6 +160,7 @@ struct clhip_ctx
     DevBuf   d_accum, d_out;
     DevBuf   d_q[2][3], d_hit, d_sq[3], d_pacc, d_gstack, d_bc, d_tot, d_ctr;
     size_t   qcap = 0;
+    uint32_t wc_stride = 0, wc_depth = 0; /* waves per row of d_ctr; depth of the last render */
     uint32_t spp  = 0;
     uint32_t blocks_trace = 0, blocks_shadow = 0, blocks_shade = 0;
     clhip_launch launch{};      /* as set; zero fields = defaults */
@@ -380,10 +381,14 @@ int ensure_render_buffers(clhip_ctx* c, size_t paths)
         CLHIP_CHECK(c, c->d_tot.alloc(sizeof(TotalCounters)));
         CLHIP_CHECK(c, hipMemsetAsync(c->d_tot.p, 0, sizeof(TotalCounters), c->stream));
     }
-    if (!c->d_ctr.p)
+    const uint32_t waves = (uint32_t)(gthreads / 64);
+    if (waves > c->wc_stride)
     {
-        CLHIP_CHECK(c, c->d_ctr.alloc(4 * sizeof(unsigned long long)));
-        CLHIP_CHECK(c, hipMemsetAsync(c->d_ctr.p, 0, 4 * sizeof(unsigned long long), c->stream));
+        if (c->d_ctr.p)
+            CLHIP_CHECK(c, hipStreamSynchronize(c->stream)); /* about to move */
+        CLHIP_CHECK(c, c->d_ctr.alloc((size_t)wc_rows(CLPT_MAXD) * waves * sizeof(unsigned long long)));
+        c->wc_stride = waves;
+        c->wc_depth  = 0; /* counts of an earlier render are gone */
     }
     return CLHIP_OK;
 }
@@ -679,7 +684,7 @@ struct BatchArgs
     BatchCounters* bc;
     TotalCounters* tot;
     uint2*         gst;
-    unsigned long long* ctr;
+    WaveCounts     wc;
     uint32_t       max_depth, blocks_trace, blocks_shadow, blocks_shade, shade_threads;
     const float*   cam_o; /* the single view's camera position (device), or null */
     GuideView      gv;
@@ -712,7 +717,7 @@ BatchArgs batch_args(clhip_ctx* c, double* accum, uint32_t max_depth, bool singl
     a.bc            = c->d_bc.as<BatchCounters>();
     a.tot           = c->d_tot.as<TotalCounters>();
     a.gst           = c->d_gstack.as<uint2>();
-    a.ctr           = c->d_ctr.as<unsigned long long>();
+    a.wc            = WaveCounts{c->d_ctr.as<unsigned long long>(), c->wc_stride};
     a.gv            = guide_view(c);
     a.guided        = guiding(c) ? 1u : 0u;
     a.blocks_guided = c->blocks_guided;
@@ -760,7 +765,7 @@ int issue_batch(clhip_ctx* c, const BatchArgs& a, bool timed)
                 CLHIP_CHECK(c, hipEventRecord(tl.a, c->stream));
             }
             if (kind == 0)
-                CLHIP_CHECK(c, clpt::launch_trace(c->stream, a.sc, qin, bc_rays(a.bc, depth), depth, a.hb, a.gst, a.ctr,
+                CLHIP_CHECK(c, clpt::launch_trace(c->stream, a.sc, qin, bc_rays(a.bc, depth), depth, a.hb, a.gst, a.wc,
                                                   depth == 1 ? a.cam_o : nullptr, a.blocks_trace));
             else if (kind == 1 && a.guided)
                 CLHIP_CHECK(c, clpt::launch_shade_guided(c->stream, a.sc, a.bt, a.gv, depth, qin, a.hb, qout, a.sq,
@@ -769,7 +774,7 @@ int issue_batch(clhip_ctx* c, const BatchArgs& a, bool timed)
                 CLHIP_CHECK(c, clpt::launch_shade(c->stream, a.sc, a.bt, depth, qin, a.hb, qout, a.sq, a.pacc, a.bc,
                                                   a.shade_threads, a.blocks_shade));
             else
-                CLHIP_CHECK(c, clpt::launch_shadow(c->stream, a.sc, a.sq, depth, a.accum, a.bc, a.gst, a.ctr,
+                CLHIP_CHECK(c, clpt::launch_shadow(c->stream, a.sc, a.sq, depth, a.accum, a.bc, a.gst, a.wc,
                                                    a.gv.nslots ? a.gv.E : nullptr, a.blocks_shadow));
             if (timed)
             {
@@ -870,8 +875,6 @@ int batch_graph(clhip_ctx* c, const BatchArgs& a, hipGraphExec_t* out)
 int run_batches(clhip_ctx* c, uint32_t nbatches, uint32_t max_depth, double* accum, bool batch_events,
                 bool single_view)
 {
-    CLHIP_CHECK(c, hipMemsetAsync(c->d_tot.p, 0, sizeof(TotalCounters), c->stream));
-    CLHIP_CHECK(c, hipMemsetAsync(c->d_ctr.p, 0, 4 * sizeof(unsigned long long), c->stream));
     recycle_events(c);
     recycle_batch_events(c);
     c->trace_launches = c->shadow_launches = 0;
@@ -895,8 +898,9 @@ int run_batches(clhip_ctx* c, uint32_t nbatches, uint32_t max_depth, double* acc
         if (rc)
             return rc;
     }
-    CLHIP_CHECK(c, clpt::launch_set_cursor(c->stream, c->d_cursor.as<uint32_t>(), 0u));
-    BatchArgs      a = batch_args(c, accum, max_depth, single_view);
+    BatchArgs a = batch_args(c, accum, max_depth, single_view);
+    CLHIP_CHECK(c, clpt::launch_render_begin(c->stream, c->d_cursor.as<uint32_t>(), a.tot, a.wc, wc_rows(max_depth)));
+    c->wc_depth      = max_depth;
     hipGraphExec_t x = nullptr;
     if (use_graph(c))
     {
@@ -2153,10 +2157,15 @@ int clhip_counters(clhip_ctx* ctx, clhip_stats* out)
     CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     if (ctx->d_tot.p)
     {
-        TotalCounters      t;
-        unsigned long long c[4];
+        TotalCounters t;
+        if (ctx->wc_depth)
+        {
+            const WaveCounts wc{ctx->d_ctr.as<unsigned long long>(), ctx->wc_stride};
+            CLHIP_CHECK(ctx, clpt::launch_sum_waves(ctx->stream, wc, wc_rows(ctx->wc_depth),
+                                                    ctx->d_tot.as<TotalCounters>()));
+            CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+        }
         CLHIP_CHECK(ctx, hipMemcpy(&t, ctx->d_tot.p, sizeof(t), hipMemcpyDeviceToHost));
-        CLHIP_CHECK(ctx, hipMemcpy(c, ctx->d_ctr.p, sizeof(c), hipMemcpyDeviceToHost));
         for (int b = 0; b <= CLHIP_MAX_DEPTH && b < CLPT_MAXD + 2; ++b)
         {
             out->rays[b]    = t.rays[b];
@@ -2164,10 +2173,10 @@ int clhip_counters(clhip_ctx* ctx, clhip_stats* out)
             out->shadow[b]  = t.shadow[b];
             out->visible[b] = t.visible[b];
         }
-        out->trace_nodes  = c[0];
-        out->trace_tris   = c[1];
-        out->shadow_nodes = c[2];
-        out->shadow_tris  = c[3];
+        out->trace_nodes  = t.trace_nodes;
+        out->trace_tris   = t.trace_tris;
+        out->shadow_nodes = t.shadow_nodes;
+        out->shadow_tris  = t.shadow_tris;
     }
     out->trace_launches  = ctx->trace_launches;
     out->shadow_launches = ctx->shadow_launches;

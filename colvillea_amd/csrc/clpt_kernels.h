@@ -13,7 +13,7 @@ namespace clpt
 hipError_t launch_camera(hipStream_t s, const BatchTable& bt, const GuideView& gv, const RayQueue& q, BatchCounters* bc,
                          uint32_t write_o, uint32_t threads, uint32_t blocks);
 hipError_t launch_trace(hipStream_t s, const SceneView& sc, const RayQueue& q, const uint32_t* count, uint32_t depth,
-                        const HitBuf& hb, uint2* gstack, unsigned long long* ctr, const float* cam_o, uint32_t blocks);
+                        const HitBuf& hb, uint2* gstack, const WaveCounts& wc, const float* cam_o, uint32_t blocks);
 hipError_t launch_shade(hipStream_t s, const SceneView& sc, const BatchTable& bt, uint32_t depth, const RayQueue& qin,
                         const HitBuf& hb, const RayQueue& qout, const ShadowQueue& sq, float* pacc, BatchCounters* bc,
                         uint32_t threads, uint32_t blocks);
@@ -22,12 +22,15 @@ hipError_t launch_shade_guided(hipStream_t s, const SceneView& sc, const BatchTa
                                uint32_t depth, const RayQueue& qin, const HitBuf& hb, const RayQueue& qout,
                                const ShadowQueue& sq, float* pacc, BatchCounters* bc, uint32_t blocks);
 hipError_t launch_shadow(hipStream_t s, const SceneView& sc, const ShadowQueue& sq, uint32_t depth, double* accum,
-                         BatchCounters* bc, uint2* gstack, unsigned long long* ctr, float4* guide_E, uint32_t blocks);
+                         BatchCounters* bc, uint2* gstack, const WaveCounts& wc, float4* guide_E, uint32_t blocks);
 /* Escaped-ray radiance of the batch's paths (3 floats per path slot, written
  * by shading) into the float64 film, one thread per pixel and view. */
 hipError_t launch_film_fold(hipStream_t s, const BatchTable& bt, const float* pacc, double* accum, uint32_t blocks);
 hipError_t launch_batch_end(hipStream_t s, const BatchCounters* bc, TotalCounters* tot, uint32_t* cursor);
-hipError_t launch_set_cursor(hipStream_t s, uint32_t* cursor, uint32_t value);
+/* Zeroes the batch cursor, the totals and the first `rows` rows of the
+ * traversal counts; and sums those rows into the totals. */
+hipError_t launch_render_begin(hipStream_t s, uint32_t* cursor, TotalCounters* tot, const WaveCounts& wc, uint32_t rows);
+hipError_t launch_sum_waves(hipStream_t s, const WaveCounts& wc, uint32_t rows, TotalCounters* tot);
 hipError_t launch_resolve(hipStream_t s, const double* accum, uint32_t npix, uint32_t spp, int srgb, float4* out);
 hipError_t launch_srgb_batch(hipStream_t s, const float* in, uint32_t n, int decode, float* out);
 hipError_t launch_texture_u8(hipStream_t s, const uchar4* in, uint32_t n, int srgb, float4* out);

@@ -49,18 +49,11 @@ __device__ __forceinline__ void wave_push2(unsigned long long* counter, bool wan
     slot_b                         = hi + (uint32_t)__popcll(mb & below);
 }
 
-__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
+/* Adds to this wave's word of a counter row (wave: its number in the grid). */
+__device__ __forceinline__ void wave_add(const WaveCounts& wc, uint32_t row, uint32_t wave, unsigned long long v)
 {
-    for (int off = 32; off > 0; off >>= 1)
-        v += __shfl_xor(v, off);
-    return v;
-}
-
-__device__ __forceinline__ void wave_count(uint32_t* counter, bool pred)
-{
-    const unsigned long long mask = __ballot(pred);
-    if (mask != 0ull && lane_id() == (uint32_t)(__ffsll((long long)mask) - 1))
-        atomicAdd(counter, (uint32_t)__popcll(mask));
+    if (v)
+        wc.c[(size_t)row * wc.stride + wave] += v;
 }
 
 /* A path's radiance from its escaped ray, kept by shading in a float32
@@ -778,8 +771,6 @@ __global__ __launch_bounds__(256) void k_camera(BatchTable bt, GuideView gv, Ray
         {
             bc->rs[2 * k]     = 0u;
             bc->rs[2 * k + 1] = 0u;
-            bc->hits[k]       = 0u;
-            bc->visible[k]    = 0u;
         }
         *bc_rays(bc, 1) = npaths;
     }
@@ -812,11 +803,10 @@ __global__ __launch_bounds__(256) void k_camera(BatchTable bt, GuideView gv, Ray
 
 template <int W>
 __global__ __launch_bounds__(256, 5) void k_trace(SceneView sc, RayQueue q, const uint32_t* count, uint32_t depth,
-                                               HitBuf hb, uint2* gstack, unsigned long long* ctr,
-                                               const float* cam_o)
+                                               HitBuf hb, uint2* gstack, WaveCounts wc, const float* cam_o)
 {
     CLPT_DECLARE_STACK(st, gstack);
-    unsigned long long sn = 0, stt = 0; /* the wave's node visits and triangle tests */
+    unsigned long long sn = 0, stt = 0, sh = 0; /* the wave's node visits, triangle tests and hits */
     const uint32_t     n    = *count;
     const float        tmin = depth == 1 ? 0.0f : CLPT_RAY_EPS;
     /* camera rays of a single view: every origin is the camera position
@@ -847,6 +837,7 @@ __global__ __launch_bounds__(256, 5) void k_trace(SceneView sc, RayQueue q, cons
         const unsigned long long mask = __ballot(fin);
         if (mask)
         {
+            sh += (unsigned long long)__popcll(__ballot(fin && tr.found));
             if (fin)
             {
                 i      = pool.take(mask);
@@ -863,8 +854,9 @@ __global__ __launch_bounds__(256, 5) void k_trace(SceneView sc, RayQueue q, cons
     }
     if (lane_id() == 0)
     {
-        atomicAdd(ctr + 0, sn);
-        atomicAdd(ctr + 1, stt);
+        wave_add(wc, CLPT_WC_TRACE_NODES, st.gid >> 6, sn);
+        wave_add(wc, CLPT_WC_TRACE_TRIS, st.gid >> 6, stt);
+        wave_add(wc, wc_hits(depth), st.gid >> 6, sh);
     }
 }
 
@@ -1044,7 +1036,6 @@ __global__ __launch_bounds__(256) void k_shade(SceneView sc, BatchTable bt, uint
             }
         }
         /* converged: wave-aggregated queue pushes */
-        wave_count(&bc->hits[depth], hit);
         uint32_t ss, ns;
         wave_push2(bc_push(bc, depth), want_shadow, want_next, ss, ns);
         if (want_shadow)
@@ -1305,7 +1296,6 @@ __global__ __launch_bounds__(256, 2) void k_shade_guided(SceneView sc, BatchTabl
                 }
             }
         }
-        wave_count(&bc->hits[depth], hit);
         uint32_t ss, ns;
         wave_push2(bc_push(bc, depth), want_shadow, want_next, ss, ns);
         if (want_shadow)
@@ -1326,8 +1316,7 @@ __global__ __launch_bounds__(256, 2) void k_shade_guided(SceneView sc, BatchTabl
 
 template <int W>
 __global__ __launch_bounds__(256, 6) void k_shadow(SceneView sc, ShadowQueue sq, uint32_t depth, double* accum,
-                                                BatchCounters* bc, uint2* gstack, unsigned long long* ctr,
-                                                float4* guide_E)
+                                                BatchCounters* bc, uint2* gstack, WaveCounts wc, float4* guide_E)
 {
     CLPT_DECLARE_STACK(st, gstack);
     unsigned long long sn = 0, stt = 0, sv = 0; /* the wave's node visits, triangle tests, unoccluded rays */
@@ -1391,10 +1380,9 @@ __global__ __launch_bounds__(256, 6) void k_shadow(SceneView sc, ShadowQueue sq,
     }
     if (lane_id() == 0)
     {
-        atomicAdd(ctr + 2, sn);
-        atomicAdd(ctr + 3, stt);
-        if (sv)
-            atomicAdd(&bc->visible[depth], (uint32_t)sv);
+        wave_add(wc, CLPT_WC_SHADOW_NODES, st.gid >> 6, sn);
+        wave_add(wc, CLPT_WC_SHADOW_TRIS, st.gid >> 6, stt);
+        wave_add(wc, wc_visible(depth), st.gid >> 6, sv);
     }
 }
 
@@ -1434,20 +1422,62 @@ __global__ void k_batch_end(const BatchCounters* bc, TotalCounters* tot, uint32_
     if (b < CLPT_MAXD + 2)
     {
         tot->rays[b] += b >= 1 ? bc->rs[2 * b - 1] : 0u;
-        tot->hits[b] += bc->hits[b];
         tot->shadow[b] += bc->rs[2 * b];
-        tot->visible[b] += bc->visible[b];
     }
     if (b == 0)
         *cursor += 1u;
 }
 
-/* Sets the batch cursor (a kernel rather than a memset, so that it may sit
- * in a captured graph). */
-__global__ void k_set_cursor(uint32_t* cursor, uint32_t value)
+/* The state a render starts from: first batch, zero totals and traversal
+ * counts (one kernel instead of a memset each; it may sit in a captured
+ * graph). */
+__global__ __launch_bounds__(256) void k_render_begin(uint32_t* cursor, TotalCounters* tot, WaveCounts wc, uint32_t rows)
 {
-    if (threadIdx.x == 0)
-        *cursor = value;
+    const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t   n   = (size_t)rows * wc.stride;
+    for (size_t i = gid; i < n; i += (size_t)gridDim.x * blockDim.x)
+        wc.c[i] = 0ull;
+    if (blockIdx.x == 0)
+    {
+        unsigned long long* t = reinterpret_cast<unsigned long long*>(tot);
+        for (uint32_t i = threadIdx.x; i < sizeof(TotalCounters) / 8u; i += blockDim.x)
+            t[i] = 0ull;
+        if (threadIdx.x == 0)
+            *cursor = 0u;
+    }
+}
+
+/* Row r = blockIdx.x of the traversal counts, summed into the totals. */
+__global__ __launch_bounds__(256) void k_sum_waves(WaveCounts wc, TotalCounters* tot)
+{
+    __shared__ unsigned long long red[256];
+    const uint32_t                r = blockIdx.x;
+    unsigned long long            v = 0;
+    for (uint32_t w = threadIdx.x; w < wc.stride; w += blockDim.x)
+        v += wc.c[(size_t)r * wc.stride + w];
+    red[threadIdx.x] = v;
+    __syncthreads();
+    for (uint32_t k = 128; k > 0; k >>= 1)
+    {
+        if (threadIdx.x < k)
+            red[threadIdx.x] += red[threadIdx.x + k];
+        __syncthreads();
+    }
+    if (threadIdx.x != 0)
+        return;
+    v = red[0];
+    if (r == CLPT_WC_TRACE_NODES)
+        tot->trace_nodes = v;
+    else if (r == CLPT_WC_TRACE_TRIS)
+        tot->trace_tris = v;
+    else if (r == CLPT_WC_SHADOW_NODES)
+        tot->shadow_nodes = v;
+    else if (r == CLPT_WC_SHADOW_TRIS)
+        tot->shadow_tris = v;
+    else if (r % 2u == 0u)
+        tot->hits[(r - 2u) / 2u] = v;
+    else
+        tot->visible[(r - 3u) / 2u] = v;
 }
 
 /* sums / spp per pixel; with srgb the display copy is encoded as the
@@ -1859,12 +1889,12 @@ hipError_t launch_camera(hipStream_t s, const BatchTable& bt, const GuideView& g
 }
 
 hipError_t launch_trace(hipStream_t s, const SceneView& sc, const RayQueue& q, const uint32_t* count, uint32_t depth,
-                        const HitBuf& hb, uint2* gstack, unsigned long long* ctr, const float* cam_o, uint32_t blocks)
+                        const HitBuf& hb, uint2* gstack, const WaveCounts& wc, const float* cam_o, uint32_t blocks)
 {
     if (sc.bvh_width == 8)
-        hipLaunchKernelGGL(k_trace<8>, dim3(blocks), dim3(256), 0, s, sc, q, count, depth, hb, gstack, ctr, cam_o);
+        hipLaunchKernelGGL(k_trace<8>, dim3(blocks), dim3(256), 0, s, sc, q, count, depth, hb, gstack, wc, cam_o);
     else
-        hipLaunchKernelGGL(k_trace<4>, dim3(blocks), dim3(256), 0, s, sc, q, count, depth, hb, gstack, ctr, cam_o);
+        hipLaunchKernelGGL(k_trace<4>, dim3(blocks), dim3(256), 0, s, sc, q, count, depth, hb, gstack, wc, cam_o);
     return hipGetLastError();
 }
 
@@ -1890,12 +1920,12 @@ hipError_t launch_shade_guided(hipStream_t s, const SceneView& sc, const BatchTa
 }
 
 hipError_t launch_shadow(hipStream_t s, const SceneView& sc, const ShadowQueue& sq, uint32_t depth, double* accum,
-                         BatchCounters* bc, uint2* gstack, unsigned long long* ctr, float4* guide_E, uint32_t blocks)
+                         BatchCounters* bc, uint2* gstack, const WaveCounts& wc, float4* guide_E, uint32_t blocks)
 {
     if (sc.bvh_width == 8)
-        hipLaunchKernelGGL(k_shadow<8>, dim3(blocks), dim3(256), 0, s, sc, sq, depth, accum, bc, gstack, ctr, guide_E);
+        hipLaunchKernelGGL(k_shadow<8>, dim3(blocks), dim3(256), 0, s, sc, sq, depth, accum, bc, gstack, wc, guide_E);
     else
-        hipLaunchKernelGGL(k_shadow<4>, dim3(blocks), dim3(256), 0, s, sc, sq, depth, accum, bc, gstack, ctr, guide_E);
+        hipLaunchKernelGGL(k_shadow<4>, dim3(blocks), dim3(256), 0, s, sc, sq, depth, accum, bc, gstack, wc, guide_E);
     return hipGetLastError();
 }
 
@@ -1911,9 +1941,16 @@ hipError_t launch_batch_end(hipStream_t s, const BatchCounters* bc, TotalCounter
     return hipGetLastError();
 }
 
-hipError_t launch_set_cursor(hipStream_t s, uint32_t* cursor, uint32_t value)
+hipError_t launch_render_begin(hipStream_t s, uint32_t* cursor, TotalCounters* tot, const WaveCounts& wc, uint32_t rows)
 {
-    hipLaunchKernelGGL(k_set_cursor, dim3(1), dim3(64), 0, s, cursor, value);
+    hipLaunchKernelGGL(k_render_begin, dim3(grid_for((uint64_t)rows * wc.stride, 256, 512)), dim3(256), 0, s, cursor, tot,
+                       wc, rows);
+    return hipGetLastError();
+}
+
+hipError_t launch_sum_waves(hipStream_t s, const WaveCounts& wc, uint32_t rows, TotalCounters* tot)
+{
+    hipLaunchKernelGGL(k_sum_waves, dim3(rows), dim3(256), 0, s, wc, tot);
     return hipGetLastError();
 }
 
