@@ -358,13 +358,14 @@ int ensure_render_buffers(clhip_ctx* c, size_t paths)
     CLHIP_CHECK(c, c->d_out.alloc(npix * sizeof(float4)));
     if (paths > c->qcap)
     {
+        const size_t slots = (size_t)CLPT_SEGS * seg_slots(paths);
         for (int q = 0; q < 2; ++q)
             for (int k = 0; k < 3; ++k)
-                CLHIP_CHECK(c, c->d_q[q][k].alloc(paths * sizeof(float4)));
-        CLHIP_CHECK(c, c->d_hit.alloc(paths * sizeof(float4)));
-        CLHIP_CHECK(c, c->d_sq[0].alloc(paths * sizeof(float4)));
-        CLHIP_CHECK(c, c->d_sq[1].alloc(paths * sizeof(float4)));
-        CLHIP_CHECK(c, c->d_sq[2].alloc(paths * sizeof(float2)));
+                CLHIP_CHECK(c, c->d_q[q][k].alloc(slots * sizeof(float4)));
+        CLHIP_CHECK(c, c->d_hit.alloc(slots * sizeof(float4)));
+        CLHIP_CHECK(c, c->d_sq[0].alloc(slots * sizeof(float4)));
+        CLHIP_CHECK(c, c->d_sq[1].alloc(slots * sizeof(float4)));
+        CLHIP_CHECK(c, c->d_sq[2].alloc(slots * sizeof(float2)));
         CLHIP_CHECK(c, c->d_pacc.alloc(paths * 3 * sizeof(float)));
         c->qcap = paths;
     }
@@ -594,13 +595,18 @@ clpt::GuideTrainBufs guide_bufs(clhip_ctx* c)
     return b;
 }
 
+/* A grid of about `blocks` blocks as the segmented queues need it: a
+ * multiple of CLPT_SEGS, not above `blocks` (a persistent grid may not
+ * exceed the resident blocks) unless that is none at all. */
+uint32_t seg_grid(uint32_t blocks) { return std::max(CLPT_SEGS, blocks / CLPT_SEGS * CLPT_SEGS); }
+
 /* Grid sizes from the launch shape (zero = default). */
 void apply_launch(clhip_ctx* c)
 {
     const clhip_launch& l = c->launch;
-    c->blocks_trace       = c->num_cus * (l.trace_blocks_per_cu ? l.trace_blocks_per_cu : c->def_trace);
-    c->blocks_shadow      = c->num_cus * (l.shadow_blocks_per_cu ? l.shadow_blocks_per_cu : c->def_shadow);
-    c->blocks_shade       = c->num_cus * (l.shade_blocks_per_cu ? l.shade_blocks_per_cu : 8u);
+    c->blocks_trace       = seg_grid(c->num_cus * (l.trace_blocks_per_cu ? l.trace_blocks_per_cu : c->def_trace));
+    c->blocks_shadow      = seg_grid(c->num_cus * (l.shadow_blocks_per_cu ? l.shadow_blocks_per_cu : c->def_shadow));
+    c->blocks_shade       = seg_grid(c->num_cus * (l.shade_blocks_per_cu ? l.shade_blocks_per_cu : 8u));
 }
 
 bool use_graph(const clhip_ctx* c) { return !c->timing && c->launch.graph != 2u; }
@@ -708,7 +714,7 @@ BatchArgs batch_args(clhip_ctx* c, double* accum, uint32_t max_depth, bool singl
         a.q[k].o     = c->d_q[k][0].as<float4>();
         a.q[k].d     = c->d_q[k][1].as<float4>();
         a.q[k].T     = c->d_q[k][2].as<float4>();
-        a.q[k].count = nullptr;
+        a.q[k].seg_cap = seg_slots(c->qcap);
     }
     a.hb            = HitBuf{c->d_hit.as<float4>()};
     a.sq            = ShadowQueue{c->d_sq[0].as<float4>(), c->d_sq[1].as<float4>(), c->d_sq[2].as<float2>(), nullptr};
@@ -765,7 +771,7 @@ int issue_batch(clhip_ctx* c, const BatchArgs& a, bool timed)
                 CLHIP_CHECK(c, hipEventRecord(tl.a, c->stream));
             }
             if (kind == 0)
-                CLHIP_CHECK(c, clpt::launch_trace(c->stream, a.sc, qin, bc_rays(a.bc, depth), depth, a.hb, a.gst, a.wc,
+                CLHIP_CHECK(c, clpt::launch_trace(c->stream, a.sc, qin, a.bc, depth, a.hb, a.gst, a.wc,
                                                   depth == 1 ? a.cam_o : nullptr, a.blocks_trace));
             else if (kind == 1 && a.guided)
                 CLHIP_CHECK(c, clpt::launch_shade_guided(c->stream, a.sc, a.bt, a.gv, depth, qin, a.hb, qout, a.sq,
@@ -774,7 +780,7 @@ int issue_batch(clhip_ctx* c, const BatchArgs& a, bool timed)
                 CLHIP_CHECK(c, clpt::launch_shade(c->stream, a.sc, a.bt, depth, qin, a.hb, qout, a.sq, a.pacc, a.bc,
                                                   a.shade_threads, a.blocks_shade));
             else
-                CLHIP_CHECK(c, clpt::launch_shadow(c->stream, a.sc, a.sq, depth, a.accum, a.bc, a.gst, a.wc,
+                CLHIP_CHECK(c, clpt::launch_shadow(c->stream, a.sc, a.sq, qin.seg_cap, depth, a.accum, a.bc, a.gst, a.wc,
                                                    a.gv.nslots ? a.gv.E : nullptr, a.blocks_shadow));
             if (timed)
             {
@@ -892,7 +898,7 @@ int run_batches(clhip_ctx* c, uint32_t nbatches, uint32_t max_depth, double* acc
     c->train_timed.clear();
     if (guiding(c))
     {
-        int rc = guide_record_buffers(c, c->guide.train ? c->guide.record_paths : 0u, c->qcap);
+        int rc = guide_record_buffers(c, c->guide.train ? c->guide.record_paths : 0u, (size_t)CLPT_SEGS * seg_slots(c->qcap));
         if (!rc && c->guide.train)
             rc = guide_train_buffers(c, c->guide.batch_size, c->guide.steps_per_batch);
         if (rc)
@@ -1118,7 +1124,7 @@ int clhip_create(uint32_t width, uint32_t height, uint32_t integrator_type, clhi
         const uint32_t ot = env_u("CLPT_TRACE_BLOCKS_PER_CU"), os = env_u("CLPT_SHADOW_BLOCKS_PER_CU");
         c->def_trace  = ot ? ot : std::max(1u, rt);
         c->def_shadow = os ? os : std::max(1u, rs);
-        c->blocks_guided = c->num_cus * std::max(1u, clpt::resident_blocks_per_cu(3));
+        c->blocks_guided = seg_grid(c->num_cus * std::max(1u, clpt::resident_blocks_per_cu(3)));
         apply_launch(c.get());
     }
     e          = hipStreamCreate(&c->stream);
@@ -2509,7 +2515,7 @@ int clhip_set_guide(clhip_ctx* ctx, const clhip_guide* g)
     {
         int rc = guide_train_buffers(ctx, v.batch_size, v.steps_per_batch);
         if (!rc)
-            rc = guide_record_buffers(ctx, v.record_paths, ctx->qcap);
+            rc = guide_record_buffers(ctx, v.record_paths, (size_t)CLPT_SEGS * seg_slots(ctx->qcap));
         if (rc)
             return rc;
     }

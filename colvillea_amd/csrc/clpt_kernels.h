@@ -6,13 +6,15 @@
 
 namespace clpt
 {
-/* `threads` per block (64, 128 or 256) for the camera and plain shading
+/* The grids of the closest-hit, shading and any-hit kernels are multiples of
+ * CLPT_SEGS blocks (block b works on queue segment b % CLPT_SEGS).
+ * `threads` per block (64, 128 or 256) for the camera and plain shading
  * kernels; write_o = 0 leaves the origin plane unwritten for a batch of one
  * view, whose closest-hit launch at depth 1 then takes cam_o (the view's
  * camera position in device memory) as every ray's origin */
 hipError_t launch_camera(hipStream_t s, const BatchTable& bt, const GuideView& gv, const RayQueue& q, BatchCounters* bc,
                          uint32_t write_o, uint32_t threads, uint32_t blocks);
-hipError_t launch_trace(hipStream_t s, const SceneView& sc, const RayQueue& q, const uint32_t* count, uint32_t depth,
+hipError_t launch_trace(hipStream_t s, const SceneView& sc, const RayQueue& q, BatchCounters* bc, uint32_t depth,
                         const HitBuf& hb, uint2* gstack, const WaveCounts& wc, const float* cam_o, uint32_t blocks);
 hipError_t launch_shade(hipStream_t s, const SceneView& sc, const BatchTable& bt, uint32_t depth, const RayQueue& qin,
                         const HitBuf& hb, const RayQueue& qout, const ShadowQueue& sq, float* pacc, BatchCounters* bc,
@@ -21,7 +23,7 @@ hipError_t launch_shade(hipStream_t s, const SceneView& sc, const BatchTable& bt
 hipError_t launch_shade_guided(hipStream_t s, const SceneView& sc, const BatchTable& bt, const GuideView& gv,
                                uint32_t depth, const RayQueue& qin, const HitBuf& hb, const RayQueue& qout,
                                const ShadowQueue& sq, float* pacc, BatchCounters* bc, uint32_t blocks);
-hipError_t launch_shadow(hipStream_t s, const SceneView& sc, const ShadowQueue& sq, uint32_t depth, double* accum,
+hipError_t launch_shadow(hipStream_t s, const SceneView& sc, const ShadowQueue& sq, uint32_t seg_cap, uint32_t depth, double* accum,
                          BatchCounters* bc, uint2* gstack, const WaveCounts& wc, float4* guide_E, uint32_t blocks);
 /* Escaped-ray radiance of the batch's paths (3 floats per path slot, written
  * by shading) into the float64 film, one thread per pixel and view. */

@@ -194,14 +194,14 @@ struct BatchTable
     uint32_t          tile; /* 1: paths of a sample in pixel rows; T > 1: in T x T tiles */
 };
 
-/* A ray queue: 3 float4 planes + count (device). */
+/* A ray queue: 3 float4 planes of CLPT_SEGS x seg_cap slots. */
 struct RayQueue
 {
     float4*   o;  /* origin.xyz, w unused (read by traversal only) */
     float4*   d;  /* direction.xyz, path id (bits) */
     float4*   T;  /* throughput.xyz, previous BSDF pdf (read by shading only; not
                      written for camera paths, whose throughput is 1 and pdf 0) */
-    uint32_t* count;
+    uint32_t  seg_cap; /* slots of a segment; segment s starts at slot s * seg_cap */
 };
 
 /* Closest hit of each ray: b1, b2, instance (bits; CLPT_NO_HIT for a miss),
@@ -217,7 +217,6 @@ struct ShadowQueue
     float4*   o; /* origin.xyz, Lo.r */
     float4*   d; /* direction.xyz, Lo.g */
     float2*   x; /* Lo.b, pixel (bits) */
-    uint32_t* count;
     uint32_t* tag; /* training record of the shadow ray (guided shading only; else NULL) */
 };
 
@@ -266,21 +265,56 @@ struct GuideView
 };
 
 #define CLPT_MAXD 32
-/* Per-batch queue counts.  The rays of depth d + 1 and the shadow rays of
- * depth d are interleaved (rs[2 d] = shadow rays of depth d, rs[2 d + 1] =
- * rays of depth d + 1), so that shading reserves both of its output queues
- * with one 64-bit atomic on &rs[2 d]. */
-struct alignas(8) BatchCounters
+/* The ray and shadow queues are CLPT_SEGS segments of seg_cap slots each,
+ * with a count of their own: shading block b reads segment b % CLPT_SEGS and
+ * appends to the same segment of the output queues, so a segment never
+ * receives more rays than it held (camera paths are dealt to the segments in
+ * windows of CLPT_SEG_WIN).  Slots are reserved by one atomic per wave, and
+ * atomics of all XCDs on one word complete one per 12.7 ns: with a single
+ * count they were the whole shading time, 1.65 ms per 8.3 M rays of a closed
+ * room.  With a count per XCD, in a line of its own (blocks are dealt to the
+ * 8 XCDs round robin, so a segment stays with one XCD), shading of a 1080p
+ * 64-spp frame takes 16.0 ms instead of 24.9 and of the room (4 spp) 7.3
+ * instead of 14.5; 16, 32 and 64 segments measure no faster than 8. */
+#define CLPT_SEGS 8u
+#define CLPT_SEG_WIN 1024u
+
+/* Queue counts of one segment in one batch.  The rays of depth d + 1 and the
+ * shadow rays of depth d are interleaved (rs[2 d] = shadow rays of depth d,
+ * rs[2 d + 1] = rays of depth d + 1), so that shading reserves both of its
+ * output queues with one 64-bit atomic on &rs[2 d]. */
+struct alignas(256) SegCounters
 {
     uint32_t rs[2 * (CLPT_MAXD + 2)];
 };
-
-/* rays of depth d >= 1, shadow rays of depth d */
-__host__ __device__ inline uint32_t* bc_rays(BatchCounters* bc, uint32_t d) { return &bc->rs[2 * d - 1]; }
-__host__ __device__ inline uint32_t* bc_shadow(BatchCounters* bc, uint32_t d) { return &bc->rs[2 * d]; }
-__host__ __device__ inline unsigned long long* bc_push(BatchCounters* bc, uint32_t d)
+struct BatchCounters
 {
-    return reinterpret_cast<unsigned long long*>(&bc->rs[2 * d]);
+    SegCounters seg[CLPT_SEGS];
+};
+
+/* The segment of window w of a batch's camera paths: each group of CLPT_SEGS
+ * consecutive windows goes to all segments once, in an order rotated by a
+ * hash of the group (unrotated, a film whose rows hold a multiple of
+ * CLPT_SEGS windows gives each segment one band of columns, which made a
+ * 512x512 16-spp frame 3.3 instead of 2.8 ms). */
+__host__ __device__ inline uint32_t seg_of_window(uint32_t w)
+{
+    return (w + ((w / CLPT_SEGS * 0x9E3779B1u) >> 24)) % CLPT_SEGS;
+}
+
+/* slots of a segment for a batch of at most `paths` paths */
+__host__ __device__ inline uint32_t seg_slots(uint64_t paths)
+{
+    const uint64_t w = (paths + CLPT_SEG_WIN - 1u) / CLPT_SEG_WIN;
+    return (uint32_t)((w + CLPT_SEGS - 1u) / CLPT_SEGS) * CLPT_SEG_WIN;
+}
+
+/* rays of depth d >= 1, shadow rays of depth d in segment s */
+__host__ __device__ inline uint32_t* bc_rays(BatchCounters* bc, uint32_t s, uint32_t d) { return &bc->seg[s].rs[2 * d - 1]; }
+__host__ __device__ inline uint32_t* bc_shadow(BatchCounters* bc, uint32_t s, uint32_t d) { return &bc->seg[s].rs[2 * d]; }
+__host__ __device__ inline unsigned long long* bc_push(BatchCounters* bc, uint32_t s, uint32_t d)
+{
+    return reinterpret_cast<unsigned long long*>(&bc->seg[s].rs[2 * d]);
 }
 
 /* A render's traversal counts, kept per wave of the persistent traversal

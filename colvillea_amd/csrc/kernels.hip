@@ -139,8 +139,11 @@ struct TraverseStack
     st.gstride = gridDim.x * blockDim.x;                                                                               \
     st.sp      = 0
 
-/* The rays of a wave's share of a persistent launch -- rays
- * w + k * stride + j (w = the wave's first global thread, j < 64) -- handed
+/* The number of this thread among the threads of its segment's blocks. */
+__device__ __forceinline__ uint32_t seg_first() { return blockIdx.x / CLPT_SEGS * blockDim.x + threadIdx.x; }
+
+/* The rays of a wave's share of its segment in a persistent launch -- rays
+ * w + k * stride + j (w = the wave's first thread in the segment, j < 64) -- handed
  * to whichever lanes finish first: one ballot per refill and a wave-uniform
  * cursor, no atomics.  A lane that draws short rays takes more of them, so
  * the wave's lanes finish together instead of waiting for the lane with the
@@ -765,35 +768,47 @@ __global__ __launch_bounds__(256) void k_camera(BatchTable bt, GuideView gv, Ray
     const BatchRec b      = bt.batches[*bt.cursor];
     const uint32_t npaths = b.npaths;
     const uint32_t tstr   = guide_tstride(gv, npaths);
-    if (gid == 0)
+    if (blockIdx.x == 0)
     {
-        for (int k = 0; k < CLPT_MAXD + 2; ++k)
+        for (uint32_t k = threadIdx.x; k < CLPT_SEGS * 2u * (CLPT_MAXD + 2u); k += blockDim.x)
+            bc->seg[k / (2u * (CLPT_MAXD + 2u))].rs[k % (2u * (CLPT_MAXD + 2u))] = 0u;
+        __syncthreads();
+        /* depth 1: the windows of whole groups are dealt to every segment,
+         * those of the last group (the last may be partly full) by their hash */
+        if (threadIdx.x < CLPT_SEGS)
         {
-            bc->rs[2 * k]     = 0u;
-            bc->rs[2 * k + 1] = 0u;
+            const uint32_t s = threadIdx.x, nw = (npaths + CLPT_SEG_WIN - 1u) / CLPT_SEG_WIN;
+            uint32_t       c = nw / CLPT_SEGS * CLPT_SEG_WIN;
+            for (uint32_t w = nw / CLPT_SEGS * CLPT_SEGS; w < nw; ++w)
+                if (seg_of_window(w) == s)
+                    c += CLPT_SEG_WIN;
+            if (nw && seg_of_window(nw - 1u) == s)
+                c -= nw * CLPT_SEG_WIN - npaths;
+            *bc_rays(bc, s, 1) = c;
         }
-        *bc_rays(bc, 1) = npaths;
     }
     for (uint32_t i = gid; i < npaths; i += gridDim.x * blockDim.x)
     {
+        const uint32_t w    = i / CLPT_SEG_WIN;
+        const uint32_t slot = seg_of_window(w) * q.seg_cap + (w / CLPT_SEGS) * CLPT_SEG_WIN + i % CLPT_SEG_WIN;
         uint32_t vi, pixel, sample;
         locate_path(bt, b, i, vi, pixel, sample);
         const ViewRec v = bt.views[vi];
         f3            o, d;
         camera_ray(v, pixel % v.width, pixel / v.width, sample, &o, &d);
         if (write_o)
-            q.o[i] = make_float4(o.x, o.y, o.z, 0.0f);
-        q.d[i] = make_float4(d.x, d.y, d.z, __uint_as_float(i));
+            q.o[slot] = make_float4(o.x, o.y, o.z, 0.0f);
+        q.d[slot] = make_float4(d.x, d.y, d.z, __uint_as_float(i));
         /* the throughput plane is not written: a camera path's throughput is
          * 1, and shading at depth 1 takes it as such */
         if (guide_records(i, tstr, *bt.cursor))
         {
-            const uint32_t slot = i / tstr;
-            const size_t   pl   = (size_t)(CLPT_MAXD + 1) * gv.nslots;
-            const float4   z    = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const uint32_t gslot = i / tstr;
+            const size_t   pl    = (size_t)(CLPT_MAXD + 1) * gv.nslots;
+            const float4   z     = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             for (uint32_t j = 1; j <= v.max_depth; ++j)
             {
-                const size_t rec = (size_t)j * gv.nslots + slot;
+                const size_t rec = (size_t)j * gv.nslots + gslot;
                 gv.V[3 * pl + rec] = z;
                 gv.E[rec]          = z;
             }
@@ -802,18 +817,22 @@ __global__ __launch_bounds__(256) void k_camera(BatchTable bt, GuideView gv, Ray
 }
 
 template <int W>
-__global__ __launch_bounds__(256, 5) void k_trace(SceneView sc, RayQueue q, const uint32_t* count, uint32_t depth,
+__global__ __launch_bounds__(256, 5) void k_trace(SceneView sc, RayQueue q, BatchCounters* bc, uint32_t depth,
                                                HitBuf hb, uint2* gstack, WaveCounts wc, const float* cam_o)
 {
     CLPT_DECLARE_STACK(st, gstack);
+    const uint32_t seg = blockIdx.x % CLPT_SEGS; /* the grid is a multiple of CLPT_SEGS */
+    q.o += (size_t)seg * q.seg_cap;
+    q.d += (size_t)seg * q.seg_cap;
+    hb.h += (size_t)seg * q.seg_cap;
     unsigned long long sn = 0, stt = 0, sh = 0; /* the wave's node visits, triangle tests and hits */
-    const uint32_t     n    = *count;
+    const uint32_t     n    = *bc_rays(bc, seg, depth);
     const float        tmin = depth == 1 ? 0.0f : CLPT_RAY_EPS;
     /* camera rays of a single view: every origin is the camera position
      * (cam_o, the view's pos), not read from the origin plane */
     const f3       co     = cam_o ? f3{cam_o[0], cam_o[1], cam_o[2]} : f3{0.0f, 0.0f, 0.0f};
-    WavePool       pool{st.gid - lane_id(), st.gstride, 64u};
-    uint32_t       i      = st.gid;
+    WavePool       pool{seg_first() - lane_id(), gridDim.x / CLPT_SEGS * blockDim.x, 64u};
+    uint32_t       i      = seg_first();
     bool           active = i < n;
     Tracer<false, W> tr;
     if (active)
@@ -860,14 +879,32 @@ __global__ __launch_bounds__(256, 5) void k_trace(SceneView sc, RayQueue q, cons
     }
 }
 
+/* The queues' planes from the first slot of segment `seg`. */
+__device__ __forceinline__ void seg_queues(uint32_t seg, RayQueue& qin, HitBuf& hb, RayQueue& qout, ShadowQueue& sq)
+{
+    const size_t off = (size_t)seg * qin.seg_cap;
+    qin.d += off;
+    qin.T += off;
+    hb.h += off;
+    qout.o += off;
+    qout.d += off;
+    qout.T += off;
+    sq.o += off;
+    sq.d += off;
+    sq.x += off;
+    if (sq.tag)
+        sq.tag += off;
+}
+
 /* Rays per thread in one class-grouping window of the shading kernel. */
 #define CLPT_SHADE_GROUP 4u
 
 __global__ __launch_bounds__(256) void k_shade(SceneView sc, BatchTable bt, uint32_t depth, RayQueue qin, HitBuf hb,
                                                RayQueue qout, ShadowQueue sq, float* pacc, BatchCounters* bc)
 {
-    const uint32_t n      = *bc_rays(bc, depth);
-    const uint32_t stride = gridDim.x * blockDim.x;
+    const uint32_t seg    = blockIdx.x % CLPT_SEGS; /* the grid is a multiple of CLPT_SEGS */
+    const uint32_t n      = *bc_rays(bc, seg, depth);
+    seg_queues(seg, qin, hb, qout, sq);
     const bool     dome   = sc.dome_index >= 0;
     const float    nl     = (float)sc.nemitters;
     const BatchRec b      = bt.batches[*bt.cursor];
@@ -885,10 +922,10 @@ __global__ __launch_bounds__(256) void k_shade(SceneView sc, BatchTable bt, uint
     __shared__ float4   sh_h[CLPT_SHADE_GROUP * 256];
     __shared__ float4   sh_d[CLPT_SHADE_GROUP * 256];
     const uint32_t      win     = CLPT_SHADE_GROUP * blockDim.x;
-    const uint32_t      wstride = gridDim.x * win;
+    const uint32_t      wstride = gridDim.x / CLPT_SEGS * win;
     /* (window, part): every thread takes the same sequence, so the barriers
      * of a window's sort are reached by the whole block */
-    for (uint32_t wbase = blockIdx.x * win, part = 0; wbase < n;)
+    for (uint32_t wbase = blockIdx.x / CLPT_SEGS * win, part = 0; wbase < n;)
     {
         if (part == 0u)
         {
@@ -1037,7 +1074,7 @@ __global__ __launch_bounds__(256) void k_shade(SceneView sc, BatchTable bt, uint
         }
         /* converged: wave-aggregated queue pushes */
         uint32_t ss, ns;
-        wave_push2(bc_push(bc, depth), want_shadow, want_next, ss, ns);
+        wave_push2(bc_push(bc, seg, depth), want_shadow, want_next, ss, ns);
         if (want_shadow)
         {
             sq.o[ss] = make_float4(p.x, p.y, p.z, Li.x);
@@ -1080,7 +1117,9 @@ __global__ __launch_bounds__(256, 2) void k_shade_guided(SceneView sc, BatchTabl
             wscl[threadIdx.x] = FP8 ? gv.scl[threadIdx.x] : 1.0f;
         __syncthreads();
     }
-    const uint32_t n      = *bc_rays(bc, depth);
+    const uint32_t seg    = blockIdx.x % CLPT_SEGS; /* the grid is a multiple of CLPT_SEGS */
+    const uint32_t n      = *bc_rays(bc, seg, depth);
+    seg_queues(seg, qin, hb, qout, sq);
     const bool     dome   = sc.dome_index >= 0;
     const float    nl     = (float)sc.nemitters;
     const BatchRec b      = bt.batches[*bt.cursor];
@@ -1089,13 +1128,13 @@ __global__ __launch_bounds__(256, 2) void k_shade_guided(SceneView sc, BatchTabl
     __shared__ uint32_t order[CLPT_SHADE_GROUP * 256]; /* blockDim.x <= 256 (launch bounds) */
     __shared__ uint32_t ncls[8];
     const uint32_t      win     = CLPT_SHADE_GROUP * blockDim.x;
-    const uint32_t      wstride = gridDim.x * win;
+    const uint32_t      wstride = gridDim.x / CLPT_SEGS * win;
     /* rays handed to threads grouped by class over windows of
      * CLPT_SHADE_GROUP x blockDim.x rays, as in k_shade: a wave then mostly
      * holds one material, and waves without a guided vertex skip the
      * network.  Every thread takes the same (window, part) sequence and
      * runs the body (the network needs the whole wave). */
-    for (uint32_t wbase = blockIdx.x * win, part = 0; wbase < n;)
+    for (uint32_t wbase = blockIdx.x / CLPT_SEGS * win, part = 0; wbase < n;)
     {
         if (part == 0u)
         {
@@ -1297,7 +1336,7 @@ __global__ __launch_bounds__(256, 2) void k_shade_guided(SceneView sc, BatchTabl
             }
         }
         uint32_t ss, ns;
-        wave_push2(bc_push(bc, depth), want_shadow, want_next, ss, ns);
+        wave_push2(bc_push(bc, seg, depth), want_shadow, want_next, ss, ns);
         if (want_shadow)
         {
             sq.o[ss]   = make_float4(si.p.x, si.p.y, si.p.z, Li.x);
@@ -1315,14 +1354,20 @@ __global__ __launch_bounds__(256, 2) void k_shade_guided(SceneView sc, BatchTabl
 }
 
 template <int W>
-__global__ __launch_bounds__(256, 6) void k_shadow(SceneView sc, ShadowQueue sq, uint32_t depth, double* accum,
+__global__ __launch_bounds__(256, 6) void k_shadow(SceneView sc, ShadowQueue sq, uint32_t seg_cap, uint32_t depth, double* accum,
                                                 BatchCounters* bc, uint2* gstack, WaveCounts wc, float4* guide_E)
 {
     CLPT_DECLARE_STACK(st, gstack);
     unsigned long long sn = 0, stt = 0, sv = 0; /* the wave's node visits, triangle tests, unoccluded rays */
-    const uint32_t     n      = *bc_shadow(bc, depth);
-    WavePool       pool{st.gid - lane_id(), st.gstride, 64u};
-    uint32_t       i      = st.gid;
+    const uint32_t     seg    = blockIdx.x % CLPT_SEGS; /* the grid is a multiple of CLPT_SEGS */
+    const uint32_t     n      = *bc_shadow(bc, seg, depth);
+    sq.o += (size_t)seg * seg_cap;
+    sq.d += (size_t)seg * seg_cap;
+    sq.x += (size_t)seg * seg_cap;
+    if (sq.tag)
+        sq.tag += (size_t)seg * seg_cap;
+    WavePool       pool{seg_first() - lane_id(), gridDim.x / CLPT_SEGS * blockDim.x, 64u};
+    uint32_t       i      = seg_first();
     bool           active = i < n;
     Tracer<true, W> tr;
     /* the ray's radiance and pixel, read with the ray so that a visible ray's
@@ -1416,15 +1461,36 @@ __global__ __launch_bounds__(256) void k_film_fold(BatchTable bt, const float* p
     }
 }
 
-__global__ void k_batch_end(const BatchCounters* bc, TotalCounters* tot, uint32_t* cursor)
+/* One block of 64 x CLPT_BE_G threads: thread (b, g) sums the segments
+ * g, g + CLPT_BE_G, ... of depth b. */
+#define CLPT_BE_G 8
+__global__ __launch_bounds__(64 * CLPT_BE_G) void k_batch_end(const BatchCounters* bc, TotalCounters* tot, uint32_t* cursor)
 {
-    const int b = threadIdx.x;
-    if (b < CLPT_MAXD + 2)
+    __shared__ uint32_t sr[CLPT_BE_G][64], ss[CLPT_BE_G][64];
+    const uint32_t      b = threadIdx.x % 64u, g = threadIdx.x / 64u;
+    uint32_t            r = 0u, h = 0u;
+    if (b < CLPT_MAXD + 2u)
+        for (uint32_t s = g; s < CLPT_SEGS; s += CLPT_BE_G)
+        {
+            r += b >= 1u ? bc->seg[s].rs[2 * b - 1] : 0u;
+            h += bc->seg[s].rs[2 * b];
+        }
+    sr[g][b] = r;
+    ss[g][b] = h;
+    __syncthreads();
+    if (g != 0u)
+        return;
+    if (b < CLPT_MAXD + 2u)
     {
-        tot->rays[b] += b >= 1 ? bc->rs[2 * b - 1] : 0u;
-        tot->shadow[b] += bc->rs[2 * b];
+        for (uint32_t k = 1; k < CLPT_BE_G; ++k)
+        {
+            r += sr[k][b];
+            h += ss[k][b];
+        }
+        tot->rays[b] += r;
+        tot->shadow[b] += h;
     }
-    if (b == 0)
+    if (b == 0u)
         *cursor += 1u;
 }
 
@@ -1888,13 +1954,13 @@ hipError_t launch_camera(hipStream_t s, const BatchTable& bt, const GuideView& g
     return hipGetLastError();
 }
 
-hipError_t launch_trace(hipStream_t s, const SceneView& sc, const RayQueue& q, const uint32_t* count, uint32_t depth,
+hipError_t launch_trace(hipStream_t s, const SceneView& sc, const RayQueue& q, BatchCounters* bc, uint32_t depth,
                         const HitBuf& hb, uint2* gstack, const WaveCounts& wc, const float* cam_o, uint32_t blocks)
 {
     if (sc.bvh_width == 8)
-        hipLaunchKernelGGL(k_trace<8>, dim3(blocks), dim3(256), 0, s, sc, q, count, depth, hb, gstack, wc, cam_o);
+        hipLaunchKernelGGL(k_trace<8>, dim3(blocks), dim3(256), 0, s, sc, q, bc, depth, hb, gstack, wc, cam_o);
     else
-        hipLaunchKernelGGL(k_trace<4>, dim3(blocks), dim3(256), 0, s, sc, q, count, depth, hb, gstack, wc, cam_o);
+        hipLaunchKernelGGL(k_trace<4>, dim3(blocks), dim3(256), 0, s, sc, q, bc, depth, hb, gstack, wc, cam_o);
     return hipGetLastError();
 }
 
@@ -1919,13 +1985,13 @@ hipError_t launch_shade_guided(hipStream_t s, const SceneView& sc, const BatchTa
     return hipGetLastError();
 }
 
-hipError_t launch_shadow(hipStream_t s, const SceneView& sc, const ShadowQueue& sq, uint32_t depth, double* accum,
+hipError_t launch_shadow(hipStream_t s, const SceneView& sc, const ShadowQueue& sq, uint32_t seg_cap, uint32_t depth, double* accum,
                          BatchCounters* bc, uint2* gstack, const WaveCounts& wc, float4* guide_E, uint32_t blocks)
 {
     if (sc.bvh_width == 8)
-        hipLaunchKernelGGL(k_shadow<8>, dim3(blocks), dim3(256), 0, s, sc, sq, depth, accum, bc, gstack, wc, guide_E);
+        hipLaunchKernelGGL(k_shadow<8>, dim3(blocks), dim3(256), 0, s, sc, sq, seg_cap, depth, accum, bc, gstack, wc, guide_E);
     else
-        hipLaunchKernelGGL(k_shadow<4>, dim3(blocks), dim3(256), 0, s, sc, sq, depth, accum, bc, gstack, wc, guide_E);
+        hipLaunchKernelGGL(k_shadow<4>, dim3(blocks), dim3(256), 0, s, sc, sq, seg_cap, depth, accum, bc, gstack, wc, guide_E);
     return hipGetLastError();
 }
 
@@ -1937,7 +2003,7 @@ hipError_t launch_film_fold(hipStream_t s, const BatchTable& bt, const float* pa
 
 hipError_t launch_batch_end(hipStream_t s, const BatchCounters* bc, TotalCounters* tot, uint32_t* cursor)
 {
-    hipLaunchKernelGGL(k_batch_end, dim3(1), dim3(64), 0, s, bc, tot, cursor);
+    hipLaunchKernelGGL(k_batch_end, dim3(1), dim3(64 * CLPT_BE_G), 0, s, bc, tot, cursor);
     return hipGetLastError();
 }
 

@@ -1,0 +1,37 @@
+"""The segmented ray and shadow queues at the sizes where the dealing of
+camera paths changes: films of one sample whose path counts lie around one
+window (1024 paths), one round of windows over all segments (8192) and one
+window more, against the oracle (counts exact, sums to the oracle's
+rounding), with the smallest shading grid too."""
+import numpy as np
+import pytest
+
+import orc
+from colvillea_amd import Integrator, IntegratorType, scenes, upload_scene
+from test_gpu_edges import _gpu_tables
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("size", [(33, 31), (32, 32), (41, 25), (8191, 1), (128, 64), (2731, 3), (709, 13)],
+                         ids=lambda s: str(s[0] * s[1]))
+def test_paths_around_a_window(size):
+    w, h = size
+    desc = scenes.make_c0(width=w, height=h, spp=1, hdri_w=64, hdri_h=32)
+    with Integrator.createIntegrator(IntegratorType.WavefrontPathTracing, w, h) as integ:
+        upload_scene(integ, desc)
+        osums = ocnt = None
+        for shade in (0, 1):
+            integ.setLaunch(shade_blocks_per_cu=shade)
+            integ.resetIterationIndex()
+            integ.render(1)
+            sums, cnt = integ.readbackSums(), integ.counters()
+            if ocnt is None:
+                osums, ocnt = orc.Scene(desc, tables=_gpu_tables(integ, desc)).render("f32", samples=(0, 1))
+            D = desc.max_depth + 1
+            for k in ("rays", "hits", "shadow", "visible"):
+                assert np.array_equal(cnt[k][:D], ocnt[k][:D]), (k, cnt[k][:D], ocnt[k][:D])
+            assert cnt["rays"][1] == w * h
+            # the oracle adds a path's radiances (at most 5 at depth 5) in
+            # float32: at most 4 roundings of 2^-24 = 2.4e-7; the film in float64
+            assert np.allclose(sums, osums, rtol=2.5e-7, atol=1e-30)
