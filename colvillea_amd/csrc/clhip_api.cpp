@@ -1603,10 +1603,21 @@ int clhip_build_tlas(clhip_ctx* ctx, const uint32_t* mesh_of_instance, const uin
     if (nbytes > 0xffffffffull)
         return fail(ctx, CLHIP_E_UNSUPPORTED, "node array of %zu bytes exceeds 4 GiB", nbytes);
     if (ctx->bvh_width == 8)
+    {
         CLHIP_CHECK(ctx, upload(ctx->d_nodes, nodes8));
+        ctx->node_bytes = nodes8.size() * sizeof(Node8);
+    }
     else
-        CLHIP_CHECK(ctx, upload(ctx->d_nodes, nodes4));
-    ctx->node_bytes = ctx->bvh_width == 8 ? nodes8.size() * sizeof(Node8) : nodes4.size() * sizeof(Node4);
+    {
+        /* uploaded as built and packed on the device */
+        Tmp raw;
+        CLHIP_CHECK(ctx, raw.from_host(nodes4.data(), nodes4.size()));
+        CLHIP_CHECK(ctx, ctx->d_nodes.alloc(std::max<size_t>(nodes4.size() * sizeof(Node4P), 16)));
+        CLHIP_CHECK(ctx, clpt::launch_pack_nodes(ctx->stream, raw.b.as<const Node4>(), (uint32_t)nodes4.size(),
+                                                 ctx->d_nodes.as<Node4P>()));
+        CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+        ctx->node_bytes = nodes4.size() * sizeof(Node4P);
+    }
     /* the records go up now, so traversal alone (clhip_trace_rays_device)
      * needs no further upload; sync_instances fills in the materials */
     CLHIP_CHECK(ctx, upload(ctx->d_inst, inst));

@@ -10,8 +10,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-/* ---- BVH4 node: 128 bytes, one L2 line pair, loaded as 8 dwordx4.
- * Child boxes are stored per axis (SoA inside the node). ---- */
+/* ---- BVH4 node as the builder makes it: float child boxes, stored per axis
+ * (SoA inside the node).  Traversal reads its packed form, Node4P. ---- */
 struct alignas(128) Node4
 {
     float    lox[4], hix[4];
@@ -21,6 +21,21 @@ struct alignas(128) Node4
     uint32_t pad[4];
 };
 static_assert(sizeof(Node4) == 128, "Node4 is two 64-byte halves");
+
+/* ---- The BVH4 node as traversal reads it: 80 bytes, five 16-byte loads
+ * instead of the float boxes' seven, packed on the device from Node4
+ * (pack_node4).  A child's planes on axis a are p[a] + q s, q a half float
+ * rounded outward after the box was widened by 2^-20 of the node's extent,
+ * which covers the rounding of the slab test's arithmetic on them: a packed
+ * box culls nothing that the float box keeps, so hits are the same bits.
+ * Empty slots hold an inverted infinite box. ---- */
+struct alignas(16) Node4P
+{
+    uint16_t pl[3][2][4]; /* [axis][lo, hi][child], half bits */
+    float    p[3], s;
+    uint32_t child[4];
+};
+static_assert(sizeof(Node4P) == 80, "Node4P is five 16-byte words");
 
 /* ---- BVH8 node: 96 bytes, read as 6 dwordx4.  Child boxes are stored
  * relative to the node's lower corner p, quantised to bytes per axis with a
@@ -130,7 +145,7 @@ struct alignas(16) EmitterRec
 /* Everything a kernel needs to find the scene; passed by value. */
 struct SceneView
 {
-    const void*        nodes; /* Node4 or Node8 array (the tree width is a kernel template argument) */
+    const void*        nodes; /* Node4P or Node8 array (the tree width is a kernel template argument) */
     const TriRec*      tris;
     const InstanceRec* inst;
     const MeshRec*     meshes;
@@ -157,7 +172,7 @@ struct SceneView
     uint32_t           world_inst; /* the instance whose mesh subtrees the top tree holds (its
                                       transform is the identity), or 0xffffffff */
     uint32_t           ninst;
-    uint32_t           bvh_width; /* 4 (Node4) or 8 (Node8) */
+    uint32_t           bvh_width; /* 4 (Node4P) or 8 (Node8) */
     uint32_t           node_bytes; /* size of the node array (below 4 GiB) */
 };
 
