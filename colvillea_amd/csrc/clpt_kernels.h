@@ -50,11 +50,13 @@ hipError_t launch_emitter_batch(hipStream_t s, const SceneView& sc, const float*
 hipError_t launch_dome_eval_batch(hipStream_t s, const SceneView& sc, const float* dir3, uint32_t n, float* le3,
                                   float* pdf);
 /* Blocks of 256 threads resident per CU for k_trace (0), k_shadow (1), k_shade (2),
- * k_shade_guided (3). */
+ * k_shade_guided (3), k_trace_rays (4). */
 uint32_t   resident_blocks_per_cu(int which);
 hipError_t launch_copy_probe(hipStream_t s, const float4* src, float4* dst, size_t n, uint32_t blocks);
-hipError_t launch_trace_batch(hipStream_t s, const SceneView& sc, const float4* rays, uint32_t n, int any, float4* out,
-                              uint32_t* prim, uint2* gstack, uint32_t blocks);
+/* Closest hit (any = 0) or any hit of n rays on `blocks` blocks of 256
+ * threads; gstack holds blocks x 256 x (stack depth - CLPT_LDS_STACK) entries. */
+hipError_t launch_trace_rays(hipStream_t s, const SceneView& sc, const float4* rays, uint32_t n, int any, float4* out,
+                             uint32_t* prim, uint2* gstack, uint32_t blocks);
 
 /* learned proposal (guide.hip) */
 struct GuideTrainBufs
@@ -87,13 +89,11 @@ struct GuideTrainBufs
 #define CLPT_GUIDE_FUSED_MAXBLK 1024u
 uint32_t guide_fused_blocks(uint32_t N, uint32_t target, uint32_t* iters);
 /* bf16 inference, or FP8 when img8 is not NULL (scales scl) */
-/* The allocation-free trace entry point: its fixed grid, the per-device
- * address of its scratch (the stacks' overflow area), and the launch. */
+/* The allocation-free trace entry point's scratch (the stacks' overflow
+ * area): the blocks of the deepest tree it holds, and its per-device address. */
 #define CLPT_NOALLOC_BLOCKS 256u
 #define CLPT_MAX_DEVICES 64
 hipError_t noalloc_scratch(int device, uint2** out);
-hipError_t launch_trace_noalloc(hipStream_t s, const SceneView& sc, const float4* rays, uint32_t n, int any,
-                                float4* out, uint32_t* prim, uint2* scratch_addr);
 hipError_t launch_guide_mixture_batch(hipStream_t s, const float* out40, const float* dir3, const float* u3, uint32_t n,
                                       float* pdf, float* smp3, float* smp_pdf);
 hipError_t launch_guide_query_batch(hipStream_t s, const float lo[3], const float inv_ext[3], const float* p3,

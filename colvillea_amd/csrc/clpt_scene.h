@@ -174,6 +174,7 @@ struct SceneView
     uint32_t           ninst;
     uint32_t           bvh_width; /* 4 (Node4P) or 8 (Node8) */
     uint32_t           node_bytes; /* size of the node array (below 4 GiB) */
+    uint32_t           stack_need; /* most stack entries a ray can hold (at most CLPT_STACK_TOTAL) */
 };
 
 /* One camera view: film size, path depth, RNG view lane, the view's offset

@@ -1,0 +1,42 @@
+"""Given-ray tracing on a persistent grid: a ray's result does not depend on
+its place or on how many rays the call holds -- one ray, the sizes around a
+wave and a block, and more rays than the grid has lanes -- for closest hit
+and any hit, on both tree widths, with tmin and tmax of each ray's own.
+(The hits themselves are checked against brute force in test_gpu_parity.)"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from colvillea_amd import Integrator, IntegratorType, scenes, upload_scene
+from colvillea_amd import _capi as capi
+from test_zz_no_alloc import rays, trace_device
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("width", [4, 8], ids=["bvh4", "bvh8"])
+def test_results_do_not_depend_on_the_batch(width):
+    desc = scenes.make_c0(width=8, height=8, spp=1, hdri_w=32, hdri_h=16)
+    n = 700001  # the largest grid has 327680 lanes
+    r = rays(desc, n, 11, 0.0)
+    rng = np.random.default_rng(12)
+    r[:, 3] = rng.choice([0.0, 1e-3, 2.0], n)
+    r[:, 7] = rng.choice([1.0, 5.0, 3.4e38], n)
+    with Integrator.createIntegrator(IntegratorType.WavefrontPathTracing, 8, 8) as integ:
+        integ.setBVHWidth(width)
+        upload_scene(integ, desc)
+        for any_hit in (False, True):
+            hit, prim = trace_device(integ, r, any_hit)
+            assert 0.05 < (hit[:, 0] > 0).mean() < 0.95
+            at = 0
+            for m in (1, 63, 64, 65, 255, 257, 30011):
+                h, p = trace_device(integ, r[at:at + m], any_hit)
+                assert np.array_equal(h.view(np.uint32), hit[at:at + m].view(np.uint32)), m
+                assert np.array_equal(p, prim[at:at + m]), m
+                at += m
+            occ = np.zeros(n, np.uint8)
+            if any_hit:
+                capi.check(capi.lib().clhip_occlusion_batch(integ.ctx, capi.fptr(r), n,
+                                                            occ.ctypes.data_as(C.POINTER(C.c_uint8))), integ.ctx)
+                assert np.array_equal(occ != 0, hit[:, 0] != 0)
