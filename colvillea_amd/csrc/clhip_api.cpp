@@ -350,12 +350,18 @@ uint32_t default_paths_per_batch(const clhip_ctx* c)
     return c->launch.paths_per_batch ? c->launch.paths_per_batch : (128u << 20);
 }
 
+/* Stack entries a lane may need beyond its LDS part in the current scene. */
+uint32_t stack_overflow(const clhip_ctx* ctx)
+{
+    return ctx->stack_need > CLPT_LDS_STACK ? ctx->stack_need - CLPT_LDS_STACK : 1u;
+}
+
 int ensure_render_buffers(clhip_ctx* c, size_t paths)
 {
     const size_t npix = (size_t)c->width * c->height;
-    const size_t gthreads = (size_t)std::max(c->blocks_trace, c->blocks_shadow) * 256;
-    if (paths > c->qcap || 3 * npix * sizeof(double) > c->d_accum.bytes ||
-        gthreads * CLPT_GSTACK_ENTRIES * sizeof(uint2) > c->d_gstack.bytes)
+    const size_t gthreads = (size_t)(c->blocks_trace + c->blocks_shadow) * 256; /* they share a launch */
+    const size_t gbytes   = gthreads * stack_overflow(c) * sizeof(uint2);
+    if (paths > c->qcap || 3 * npix * sizeof(double) > c->d_accum.bytes || gbytes > c->d_gstack.bytes)
         CLHIP_CHECK(c, hipStreamSynchronize(c->stream)); /* buffers about to move may be in use */
     CLHIP_CHECK(c, c->d_accum.alloc(3 * npix * sizeof(double)));
     CLHIP_CHECK(c, c->d_out.alloc(npix * sizeof(float4)));
@@ -372,7 +378,7 @@ int ensure_render_buffers(clhip_ctx* c, size_t paths)
         CLHIP_CHECK(c, c->d_pacc.alloc(paths * 3 * sizeof(float)));
         c->qcap = paths;
     }
-    CLHIP_CHECK(c, c->d_gstack.alloc(gthreads * CLPT_GSTACK_ENTRIES * sizeof(uint2)));
+    CLHIP_CHECK(c, c->d_gstack.alloc(gbytes));
     if (!c->d_cursor.p)
         CLHIP_CHECK(c, c->d_cursor.alloc(256));
     if (!c->d_bc.p)
@@ -385,7 +391,7 @@ int ensure_render_buffers(clhip_ctx* c, size_t paths)
         CLHIP_CHECK(c, c->d_tot.alloc(sizeof(TotalCounters)));
         CLHIP_CHECK(c, hipMemsetAsync(c->d_tot.p, 0, sizeof(TotalCounters), c->stream));
     }
-    const uint32_t waves = (uint32_t)(gthreads / 64);
+    const uint32_t waves = std::max(c->blocks_trace, c->blocks_shadow) * 4u;
     if (waves > c->wc_stride)
     {
         if (c->d_ctr.p)
@@ -757,11 +763,14 @@ int issue_batch(clhip_ctx* c, const BatchArgs& a, bool timed)
 {
     CLHIP_CHECK(c, clpt::launch_camera(c->stream, a.bt, a.gv, a.q[0], a.bc, a.cam_o ? 0u : 1u, a.shade_threads,
                                        a.blocks_shade));
+    float4* const guide_E = a.gv.nslots ? a.gv.E : nullptr;
     for (uint32_t depth = 1; depth <= a.max_depth; ++depth)
     {
         const RayQueue& qin  = a.q[(depth - 1) & 1];
         const RayQueue& qout = a.q[depth & 1];
-        for (int kind = 0; kind < 3; ++kind)
+        /* closest hit and any hit in launches of their own while they are
+         * timed apart; else depth's shadow rays go with depth + 1's rays */
+        for (int kind = timed || depth == 1u ? 0 : 1; kind < 3; ++kind)
         {
             if (kind == 2 && depth == a.max_depth)
                 break;
@@ -782,9 +791,12 @@ int issue_batch(clhip_ctx* c, const BatchArgs& a, bool timed)
             else if (kind == 1)
                 CLHIP_CHECK(c, clpt::launch_shade(c->stream, a.sc, a.bt, depth, qin, a.hb, qout, a.sq, a.pacc, a.bc,
                                                   a.shade_threads, a.blocks_shade));
-            else
+            else if (timed)
                 CLHIP_CHECK(c, clpt::launch_shadow(c->stream, a.sc, a.sq, qin.seg_cap, depth, a.accum, a.bc, a.gst, a.wc,
-                                                   a.gv.nslots ? a.gv.E : nullptr, a.blocks_shadow));
+                                                   guide_E, a.blocks_shadow));
+            else
+                CLHIP_CHECK(c, clpt::launch_trace_shadow(c->stream, a.sc, qout, a.bc, depth, a.hb, a.sq, a.accum, a.gst,
+                                                         a.wc, guide_E, a.blocks_trace, a.blocks_shadow));
             if (timed)
             {
                 CLHIP_CHECK(c, hipEventRecord(tl.b, c->stream));
@@ -2356,12 +2368,6 @@ int clhip_dome_tables(clhip_ctx* ctx, float* pcond, float* cdfcond, float* pv, f
     if (cdfv)
         CLHIP_CHECK(ctx, hipMemcpy(cdfv, ctx->d_cdfv.p, ((size_t)ctx->dome_h + 1) * 4, hipMemcpyDeviceToHost));
     return CLHIP_OK;
-}
-
-/* Stack entries a lane may need beyond its LDS part in the current scene. */
-static uint32_t stack_overflow(const clhip_ctx* ctx)
-{
-    return ctx->stack_need > CLPT_LDS_STACK ? ctx->stack_need - CLPT_LDS_STACK : 1u;
 }
 
 /* Blocks for n given rays: a thread per ray up to full residency, and as

@@ -25,6 +25,11 @@ hipError_t launch_shade_guided(hipStream_t s, const SceneView& sc, const BatchTa
                                const ShadowQueue& sq, float* pacc, BatchCounters* bc, uint32_t blocks);
 hipError_t launch_shadow(hipStream_t s, const SceneView& sc, const ShadowQueue& sq, uint32_t seg_cap, uint32_t depth, double* accum,
                          BatchCounters* bc, uint2* gstack, const WaveCounts& wc, float4* guide_E, uint32_t blocks);
+/* The closest-hit rays of depth + 1 (queue q) and the shadow rays of depth
+ * in one launch; gstack holds the overflow of both grids' lanes. */
+hipError_t launch_trace_shadow(hipStream_t s, const SceneView& sc, const RayQueue& q, BatchCounters* bc, uint32_t depth,
+                               const HitBuf& hb, const ShadowQueue& sq, double* accum, uint2* gstack, const WaveCounts& wc,
+                               float4* guide_E, uint32_t blocks_trace, uint32_t blocks_shadow);
 /* Escaped-ray radiance of the batch's paths (3 floats per path slot, written
  * by shading) into the float64 film, one thread per pixel and view. */
 hipError_t launch_film_fold(hipStream_t s, const BatchTable& bt, const float* pacc, double* accum, uint32_t blocks);

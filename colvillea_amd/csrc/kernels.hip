@@ -4,12 +4,13 @@
  * Pipeline of one batch of paths (replaces the 30 synchronous launches per
  * spp of WavefrontPathTracingIntegrator::render, path.cpp:84-231):
  *   k_camera                         generateCameraRays (raygeneration.cu:59-103)
+ *   k_trace   closest hit, depth 1   OptiX primaryRay raygen + closest-hit/miss (optix.cu:38-75, 112-262)
  *   for depth = 1..max_depth:
- *     k_trace   closest hit          OptiX primaryRay raygen + closest-hit/miss (optix.cu:38-75, 112-262)
  *     k_shade   escape + NEE + BSDF  evaluateEscapedRays (raygeneration.cu:105-136) and
  *                                    evaluateMaterialsAndLightsPathTracing (:285-456)
- *     k_shadow  any hit + accumulate OptiX shadowRay raygen + miss (optix.cu:77-110, 265-284)
- *   k_batch_end                      per-batch counters -> totals
+ *     k_trace_shadow (not at the last depth): closest hit of depth + 1, and
+ *               any hit + accumulate OptiX shadowRay raygen + miss (optix.cu:77-110, 265-284)
+ *   k_film_fold, k_batch_end         escaped radiance -> film, counters -> totals
  * All kernels are grid-stride loops over device-side queue counts, so a
  * batch needs no host synchronisation (the reference resets counters with
  * <<<1,1>>> launches and synchronises after each kernel, cudadevice.h:185-219).
@@ -140,18 +141,14 @@ struct TraverseStack
     }
 };
 
-#define CLPT_DECLARE_STACK(st, gstack)                                                                                 \
-    __shared__ uint2 lds_stack_[CLPT_LDS_STACK * CLPT_TRACE_BLOCK];                                                    \
-    TraverseStack    st;                                                                                               \
-    st.lds     = (lds_char*)lds_stack_;                                                                                \
+#define CLPT_DECLARE_STACK(st, lds_stack, gstack)                                                                      \
+    TraverseStack st;                                                                                                  \
+    st.lds     = (lds_char*)(lds_stack);                                                                               \
     st.gmem    = (gstack);                                                                                             \
     st.gid     = blockIdx.x * CLPT_TRACE_BLOCK + threadIdx.x;                                                          \
     st.gstride = gridDim.x * CLPT_TRACE_BLOCK;                                                                         \
     st.limit   = (int)sc.stack_need * CLPT_STACK_ROW;                                                                  \
     st.reset()
-
-/* The number of this thread among the threads of its segment's blocks. */
-__device__ __forceinline__ uint32_t seg_first() { return blockIdx.x / CLPT_SEGS * blockDim.x + threadIdx.x; }
 
 /* The rays of a wave's share of its segment in a persistent launch -- rays
  * w + k * stride + j (w = the wave's first thread in the segment, j < 64) -- handed
@@ -830,12 +827,22 @@ __global__ __launch_bounds__(256) void k_camera(BatchTable bt, GuideView gv, Ray
     }
 }
 
-template <int W>
-__global__ __launch_bounds__(256, 5) void k_trace(SceneView sc, RayQueue q, BatchCounters* bc, uint32_t depth,
-                                               HitBuf hb, uint2* gstack, WaveCounts wc, const float* cam_o)
+/* LDS of a traversal block (the any-hit rays use the stack only). */
+struct TraceShared
 {
-    CLPT_DECLARE_STACK(st, gstack);
-    const uint32_t seg = blockIdx.x % CLPT_SEGS; /* the grid is a multiple of CLPT_SEGS */
+    uint2  stack[CLPT_LDS_STACK * CLPT_TRACE_BLOCK];
+    float4 ring_a[CLPT_TRACE_BLOCK]; /* d.xyz, o.x */
+    float2 ring_b[CLPT_TRACE_BLOCK]; /* o.yz */
+};
+
+/* Block bx of gx (a multiple of CLPT_SEGS) of the closest-hit rays of a
+ * depth. */
+template <int W>
+__device__ __forceinline__ void trace_block(TraceShared& sm, TraverseStack& st, uint32_t bx, uint32_t gx,
+                                            const SceneView& sc, RayQueue q, BatchCounters* bc, uint32_t depth, HitBuf hb,
+                                            const WaveCounts& wc, const float* cam_o)
+{
+    const uint32_t seg = bx % CLPT_SEGS, first = bx / CLPT_SEGS * CLPT_TRACE_BLOCK + threadIdx.x;
     q.o += (size_t)seg * q.seg_cap;
     q.d += (size_t)seg * q.seg_cap;
     hb.h += (size_t)seg * q.seg_cap;
@@ -851,13 +858,11 @@ __global__ __launch_bounds__(256, 5) void k_trace(SceneView sc, RayQueue q, Batc
      * this kernel's time at 1080p 64 spp, 3.5% in the closed room, 5% for a
      * 512x512 frame).  A lane that finds the chunk used up waits for the next
      * step. */
-    __shared__ float4 ring_a[256]; /* d.xyz, o.x */
-    __shared__ float2 ring_b[256]; /* o.yz */
     const uint32_t    rl     = threadIdx.x & ~63u;
-    const uint32_t    stride = gridDim.x / CLPT_SEGS * blockDim.x;
-    uint32_t          cbase  = (uint32_t)__builtin_amdgcn_readfirstlane((int)(seg_first() - lane_id())); /* this chunk */
+    const uint32_t    stride = gx / CLPT_SEGS * CLPT_TRACE_BLOCK;
+    uint32_t          cbase  = (uint32_t)__builtin_amdgcn_readfirstlane((int)(first - lane_id())); /* this chunk */
     uint32_t          used   = 64u; /* rays of it taken (the first go to the lanes directly) */
-    uint32_t          i      = seg_first();
+    uint32_t          i      = first;
     bool              active = i < n;
     Tracer<false, W>  tr;
     if (active)
@@ -893,8 +898,8 @@ __global__ __launch_bounds__(256, 5) void k_trace(SceneView sc, RayQueue q, Batc
                 {
                     const float4 d      = q.d[k];
                     const float4 o      = cam_o ? make_float4(co.x, co.y, co.z, 0.0f) : q.o[k];
-                    ring_a[threadIdx.x] = make_float4(d.x, d.y, d.z, o.x);
-                    ring_b[threadIdx.x] = make_float2(o.y, o.z);
+                    sm.ring_a[threadIdx.x] = make_float4(d.x, d.y, d.z, o.x);
+                    sm.ring_b[threadIdx.x] = make_float2(o.y, o.z);
                 }
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             }
@@ -905,8 +910,8 @@ __global__ __launch_bounds__(256, 5) void k_trace(SceneView sc, RayQueue q, Batc
                 active           = j < 64u && i < n;
                 if (active)
                 {
-                    const float4 a = ring_a[rl + j];
-                    const float2 b = ring_b[rl + j];
+                    const float4 a = sm.ring_a[rl + j];
+                    const float2 b = sm.ring_b[rl + j];
                     tr.start(sc, st, f3{a.w, b.x, b.y}, f3{a.x, a.y, a.z}, CLPT_FLT_MAX);
                 }
             }
@@ -915,10 +920,19 @@ __global__ __launch_bounds__(256, 5) void k_trace(SceneView sc, RayQueue q, Batc
     }
     if (lane_id() == 0)
     {
-        wave_add(wc, CLPT_WC_TRACE_NODES, st.gid >> 6, sn);
-        wave_add(wc, CLPT_WC_TRACE_TRIS, st.gid >> 6, stt);
-        wave_add(wc, wc_hits(depth), st.gid >> 6, sh);
+        wave_add(wc, CLPT_WC_TRACE_NODES, (bx * CLPT_TRACE_BLOCK + threadIdx.x) >> 6, sn);
+        wave_add(wc, CLPT_WC_TRACE_TRIS, (bx * CLPT_TRACE_BLOCK + threadIdx.x) >> 6, stt);
+        wave_add(wc, wc_hits(depth), (bx * CLPT_TRACE_BLOCK + threadIdx.x) >> 6, sh);
     }
+}
+
+template <int W>
+__global__ __launch_bounds__(CLPT_TRACE_BLOCK, 5) void k_trace(SceneView sc, RayQueue q, BatchCounters* bc, uint32_t depth,
+                                                               HitBuf hb, uint2* gstack, WaveCounts wc, const float* cam_o)
+{
+    __shared__ TraceShared sm;
+    CLPT_DECLARE_STACK(st, sm.stack, gstack);
+    trace_block<W>(sm, st, blockIdx.x, gridDim.x, sc, q, bc, depth, hb, wc, cam_o);
 }
 
 /* The queues' planes from the first slot of segment `seg`. */
@@ -1395,21 +1409,23 @@ __global__ __launch_bounds__(256, 2) void k_shade_guided(SceneView sc, BatchTabl
     }
 }
 
+/* Block bx of gx (a multiple of CLPT_SEGS) of the shadow rays of a depth:
+ * visible ones add their radiance to the film. */
 template <int W>
-__global__ __launch_bounds__(256, 6) void k_shadow(SceneView sc, ShadowQueue sq, uint32_t seg_cap, uint32_t depth, double* accum,
-                                                BatchCounters* bc, uint2* gstack, WaveCounts wc, float4* guide_E)
+__device__ __forceinline__ void shadow_block(TraverseStack& st, uint32_t bx, uint32_t gx, const SceneView& sc, ShadowQueue sq,
+                                             uint32_t seg_cap, uint32_t depth, double* accum, BatchCounters* bc,
+                                             const WaveCounts& wc, float4* guide_E)
 {
-    CLPT_DECLARE_STACK(st, gstack);
     unsigned long long sn = 0, stt = 0, sv = 0; /* the wave's node visits, triangle tests, unoccluded rays */
-    const uint32_t     seg    = blockIdx.x % CLPT_SEGS; /* the grid is a multiple of CLPT_SEGS */
+    const uint32_t     seg = bx % CLPT_SEGS, first = bx / CLPT_SEGS * CLPT_TRACE_BLOCK + threadIdx.x;
     const uint32_t     n      = *bc_shadow(bc, seg, depth);
     sq.o += (size_t)seg * seg_cap;
     sq.d += (size_t)seg * seg_cap;
     sq.x += (size_t)seg * seg_cap;
     if (sq.tag)
         sq.tag += (size_t)seg * seg_cap;
-    WavePool       pool{seg_first() - lane_id(), gridDim.x / CLPT_SEGS * blockDim.x, 64u};
-    uint32_t       i      = seg_first();
+    WavePool       pool{first - lane_id(), gx / CLPT_SEGS * CLPT_TRACE_BLOCK, 64u};
+    uint32_t       i      = first;
     bool           active = i < n;
     Tracer<true, W> tr;
     /* the ray's radiance and pixel, read with the ray so that a visible ray's
@@ -1467,10 +1483,38 @@ __global__ __launch_bounds__(256, 6) void k_shadow(SceneView sc, ShadowQueue sq,
     }
     if (lane_id() == 0)
     {
-        wave_add(wc, CLPT_WC_SHADOW_NODES, st.gid >> 6, sn);
-        wave_add(wc, CLPT_WC_SHADOW_TRIS, st.gid >> 6, stt);
-        wave_add(wc, wc_visible(depth), st.gid >> 6, sv);
+        wave_add(wc, CLPT_WC_SHADOW_NODES, (bx * CLPT_TRACE_BLOCK + threadIdx.x) >> 6, sn);
+        wave_add(wc, CLPT_WC_SHADOW_TRIS, (bx * CLPT_TRACE_BLOCK + threadIdx.x) >> 6, stt);
+        wave_add(wc, wc_visible(depth), (bx * CLPT_TRACE_BLOCK + threadIdx.x) >> 6, sv);
     }
+}
+
+template <int W>
+__global__ __launch_bounds__(CLPT_TRACE_BLOCK, 6) void k_shadow(SceneView sc, ShadowQueue sq, uint32_t seg_cap, uint32_t depth,
+                                                                double* accum, BatchCounters* bc, uint2* gstack,
+                                                                WaveCounts wc, float4* guide_E)
+{
+    __shared__ uint2 lds_stack[CLPT_LDS_STACK * CLPT_TRACE_BLOCK];
+    CLPT_DECLARE_STACK(st, lds_stack, gstack);
+    shadow_block<W>(st, blockIdx.x, gridDim.x, sc, sq, seg_cap, depth, accum, bc, wc, guide_E);
+}
+
+/* The closest-hit rays of depth + 1 (blocks 0 .. gt-1) and the shadow rays
+ * of depth (the rest) in one launch: both need only the shading of depth.
+ * A traversal launch ends with its longest ray, 50-110 us of mostly idle
+ * chip; this way the two share one tail, and shadow blocks fill the CUs as
+ * closest-hit blocks end. */
+template <int W>
+__global__ __launch_bounds__(CLPT_TRACE_BLOCK, 5) void k_trace_shadow(SceneView sc, RayQueue q, BatchCounters* bc, uint32_t depth,
+                                                                      HitBuf hb, ShadowQueue sq, double* accum, uint2* gstack,
+                                                                      WaveCounts wc, float4* guide_E, uint32_t gt)
+{
+    __shared__ TraceShared sm;
+    CLPT_DECLARE_STACK(st, sm.stack, gstack);
+    if (blockIdx.x < gt)
+        trace_block<W>(sm, st, blockIdx.x, gt, sc, q, bc, depth + 1u, hb, wc, nullptr);
+    else
+        shadow_block<W>(st, blockIdx.x - gt, gridDim.x - gt, sc, sq, q.seg_cap, depth, accum, bc, wc, guide_E);
 }
 
 /* The batch's path sums (path_set) into the film: for each entry, one thread
@@ -1889,7 +1933,8 @@ template <bool ANY, int W>
 __global__ __launch_bounds__(256, 5) void k_trace_rays(SceneView sc, const float4* rays, uint32_t n, float4* out,
                                                        uint32_t* prim, uint2* gstack)
 {
-    CLPT_DECLARE_STACK(st, gstack);
+    __shared__ uint2 lds_stack[CLPT_LDS_STACK * CLPT_TRACE_BLOCK];
+    CLPT_DECLARE_STACK(st, lds_stack, gstack);
     WavePool       pool{st.gid - lane_id(), st.gstride, 64u};
     uint32_t       i      = st.gid;
     bool           active = i < n;
@@ -2060,6 +2105,19 @@ hipError_t launch_shadow(hipStream_t s, const SceneView& sc, const ShadowQueue& 
         hipLaunchKernelGGL(k_shadow<8>, dim3(blocks), dim3(256), 0, s, sc, sq, seg_cap, depth, accum, bc, gstack, wc, guide_E);
     else
         hipLaunchKernelGGL(k_shadow<4>, dim3(blocks), dim3(256), 0, s, sc, sq, seg_cap, depth, accum, bc, gstack, wc, guide_E);
+    return hipGetLastError();
+}
+
+hipError_t launch_trace_shadow(hipStream_t s, const SceneView& sc, const RayQueue& q, BatchCounters* bc, uint32_t depth,
+                               const HitBuf& hb, const ShadowQueue& sq, double* accum, uint2* gstack, const WaveCounts& wc,
+                               float4* guide_E, uint32_t blocks_trace, uint32_t blocks_shadow)
+{
+    if (sc.bvh_width == 8)
+        hipLaunchKernelGGL(k_trace_shadow<8>, dim3(blocks_trace + blocks_shadow), dim3(256), 0, s, sc, q, bc, depth, hb, sq,
+                           accum, gstack, wc, guide_E, blocks_trace);
+    else
+        hipLaunchKernelGGL(k_trace_shadow<4>, dim3(blocks_trace + blocks_shadow), dim3(256), 0, s, sc, q, bc, depth, hb, sq,
+                           accum, gstack, wc, guide_E, blocks_trace);
     return hipGetLastError();
 }
 
