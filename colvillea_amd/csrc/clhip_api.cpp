@@ -130,7 +130,7 @@ struct clhip_ctx
     std::vector<MeshBuild>   mesh_builds; /* per-mesh trees, reassembled on every BLAS (re)build */
     uint64_t                 blas_builds = 0; /* mesh trees built since creation */
     bool                     have_blas = false, have_tlas = false;
-    DevBuf                   d_nodes, d_tris, d_meshes, d_pos, d_nrm, d_tan, d_uv, d_idx, d_inst;
+    DevBuf                   d_nodes, d_tris, d_meshes, d_shade, d_tan, d_idx, d_inst;
     size_t                   node_bytes = 0, tri_bytes = 0; /* in use in d_nodes, d_tris */
     uint2*                   noalloc_stack = nullptr; /* this device's scratch of clhip_trace_rays_device */
     std::vector<InstanceRec> inst;
@@ -280,10 +280,8 @@ SceneView scene_view(const clhip_ctx* c)
     s.node_bytes = (uint32_t)std::min<size_t>(c->node_bytes, 0xffffffffu);
     s.inst       = c->d_inst.as<const InstanceRec>();
     s.meshes     = c->d_meshes.as<const MeshRec>();
-    s.pos        = c->d_pos.as<const float>();
-    s.nrm        = c->d_nrm.as<const float>();
+    s.shade      = c->d_shade.as<const ShadeRec>();
     s.tan        = c->d_tan.as<const float>();
-    s.uv         = c->d_uv.as<const float>();
     s.idx        = c->d_idx.as<const uint32_t>();
     s.mtl        = c->d_mtl.as<const MaterialRec>();
     s.tex        = c->d_texrec.as<const TexRec>();
@@ -331,6 +329,7 @@ int sync_instances(clhip_ctx* c)
         if (m >= c->mtl.size())
             return fail(c, CLHIP_E_STATE, "instance %zu needs material %u but only %zu are built", i, m, c->mtl.size());
         c->inst[i].material = m;
+        c->inst[i].mtl_type = c->mtl[m].type;
         c->inst[i].entity   = e;
     }
     CLHIP_CHECK(c, upload(c->d_inst, c->inst));
@@ -1443,11 +1442,20 @@ static int assemble_blas(clhip_ctx* ctx)
     CLHIP_CHECK(ctx, upload(ctx->d_tris, tris));
     ctx->tri_bytes = tris.size() * sizeof(TriRec);
     CLHIP_CHECK(ctx, upload(ctx->d_meshes, recs));
-    CLHIP_CHECK(ctx, upload(ctx->d_pos, pos));
-    CLHIP_CHECK(ctx, upload(ctx->d_nrm, nrm));
     CLHIP_CHECK(ctx, upload(ctx->d_tan, tan));
-    CLHIP_CHECK(ctx, upload(ctx->d_uv, uv));
     CLHIP_CHECK(ctx, upload(ctx->d_idx, idx));
+    {
+        DevBuf d_pos, d_nrm, d_uv; /* read by the shading records' build only */
+        CLHIP_CHECK(ctx, upload(d_pos, pos));
+        CLHIP_CHECK(ctx, upload(d_nrm, nrm));
+        CLHIP_CHECK(ctx, upload(d_uv, uv));
+        CLHIP_CHECK(ctx, ctx->d_shade.alloc(std::max<size_t>(tris.size() * sizeof(ShadeRec), 16)));
+        for (const MeshRec& me : recs)
+            CLHIP_CHECK(ctx, clpt::launch_shade_recs(ctx->stream, me, ctx->d_idx.as<const uint32_t>(), d_pos.as<const float>(),
+                                                     d_nrm.as<const float>(), d_uv.as<const float>(),
+                                                     ctx->d_shade.as<ShadeRec>()));
+        CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    }
     ctx->blas_nodes4 = std::move(nodes4);
     ctx->blas_nodes8 = std::move(nodes8);
     ctx->meshes      = std::move(infos);
@@ -1527,6 +1535,10 @@ int clhip_build_tlas(clhip_ctx* ctx, const uint32_t* mesh_of_instance, const uin
                 return fail(ctx, CLHIP_E_INVALID, "instance %u: singular transform", i);
         r.blas_root = ctx->meshes[m].root;
         r.mesh      = m;
+        r.shade_off  = ctx->mesh_recs[m].idx_off;
+        r.mesh_flags = ctx->mesh_recs[m].flags;
+        r.mtl_type   = 0;
+        r.pad        = 0;
         r.material  = 0;
         r.entity    = instance_ids ? instance_ids[i] : i;
         ent[i]      = r.entity;

@@ -84,7 +84,7 @@ struct TriRec
     float4 v2;
 };
 
-struct InstanceRec
+struct alignas(16) InstanceRec
 {
     float    xf[12];  /* object -> world */
     float    inv[12]; /* world -> object */
@@ -92,7 +92,25 @@ struct InstanceRec
     uint32_t mesh;
     uint32_t material;
     uint32_t entity;
+    uint32_t shade_off;  /* the mesh's first ShadeRec */
+    uint32_t mesh_flags; /* MESH_HAS_* */
+    uint32_t mtl_type;   /* the material's type */
+    uint32_t pad;
 };
+static_assert(sizeof(InstanceRec) == 128, "InstanceRec is one 128-byte line");
+
+/* What shading reads of a hit triangle, in original triangle order: vertex
+ * positions, normals and uvs (zeros where the mesh has none) in one 128-byte
+ * line, built on the device from the indexed arrays.  Through the arrays a
+ * hit read its indices and then six places of vertices. */
+struct alignas(128) ShadeRec
+{
+    float p[3][3];
+    float n[3][3];
+    float uv[3][2];
+    float pad[8];
+};
+static_assert(sizeof(ShadeRec) == 128, "ShadeRec is one 128-byte line");
 
 enum : uint32_t
 {
@@ -149,10 +167,8 @@ struct SceneView
     const TriRec*      tris;
     const InstanceRec* inst;
     const MeshRec*     meshes;
-    const float*       pos; /* xyz per vertex */
-    const float*       nrm;
-    const float*       tan;
-    const float*       uv;
+    const ShadeRec*    shade; /* per triangle of every mesh */
+    const float*       tan;   /* xyz per vertex, read through idx */
     const uint32_t*    idx;
     const MaterialRec* mtl;
     const TexRec*      tex; /* material textures by id */

@@ -535,21 +535,19 @@ struct Surface
 __device__ __forceinline__ void surface_interaction(const SceneView& sc, const HitRec& h, Surface& si)
 {
     const InstanceRec* ip = sc.inst + h.inst;
-    const MeshRec      me = sc.meshes[ip->mesh];
-    const uint32_t     i0 = sc.idx[3 * (size_t)(me.idx_off + h.prim) + 0] + me.vtx_off;
-    const uint32_t     i1 = sc.idx[3 * (size_t)(me.idx_off + h.prim) + 1] + me.vtx_off;
-    const uint32_t     i2 = sc.idx[3 * (size_t)(me.idx_off + h.prim) + 2] + me.vtx_off;
+    const ShadeRec*    sr = sc.shade + (size_t)(ip->shade_off + h.prim);
+    const float4*      sv = reinterpret_cast<const float4*>(sr);
+    const float4       q0 = sv[0], q1 = sv[1], q2 = sv[2], q3 = sv[3], q4 = sv[4];
+    const uint32_t     mf = ip->mesh_flags;
     const float        b1 = h.b1, b2 = h.b2;
     const float        b0 = 1.0f - b1 - b2;
-    const f3 p0 = ld3(sc.pos + 3 * (size_t)i0), p1 = ld3(sc.pos + 3 * (size_t)i1), p2 = ld3(sc.pos + 3 * (size_t)i2);
+    const f3           p0{q0.x, q0.y, q0.z}, p1{q0.w, q1.x, q1.y}, p2{q1.z, q1.w, q2.x};
     const f3 po = add3(add3(sclL3(b0, p0), sclL3(b1, p1)), sclL3(b2, p2));
-    if (me.flags & MESH_HAS_UVS)
+    if (mf & MESH_HAS_UVS)
     {
-        const float* t0 = sc.uv + 2 * (size_t)i0;
-        const float* t1 = sc.uv + 2 * (size_t)i1;
-        const float* t2 = sc.uv + 2 * (size_t)i2;
-        si.u            = b0 * t0[0] + b1 * t1[0] + b2 * t2[0];
-        si.v            = b0 * t0[1] + b1 * t1[1] + b2 * t2[1];
+        const float4 q5 = sv[5]; /* uvs from q4.z on */
+        si.u            = b0 * q4.z + b1 * q5.x + b2 * q5.z;
+        si.v            = b0 * q4.w + b1 * q5.y + b2 * q5.w;
     }
     else
     {
@@ -558,13 +556,17 @@ __device__ __forceinline__ void surface_interaction(const SceneView& sc, const H
     }
     const f3 ngo = cross3(sub3(p1, p0), sub3(p2, p0));
     f3       nso = ngo;
-    if (me.flags & MESH_HAS_NORMALS)
-        nso = add3(add3(sclL3(b0, ld3(sc.nrm + 3 * (size_t)i0)), sclL3(b1, ld3(sc.nrm + 3 * (size_t)i1))),
-                   sclL3(b2, ld3(sc.nrm + 3 * (size_t)i2)));
+    if (mf & MESH_HAS_NORMALS)
+        nso = add3(add3(sclL3(b0, f3{q2.y, q2.z, q2.w}), sclL3(b1, f3{q3.x, q3.y, q3.z})), sclL3(b2, f3{q3.w, q4.x, q4.y}));
     f3 tgo{0.0f, 0.0f, 0.0f};
-    if (me.flags & MESH_HAS_TANGENTS)
-        tgo = add3(add3(sclL3(b0, ld3(sc.tan + 3 * (size_t)i0)), sclL3(b1, ld3(sc.tan + 3 * (size_t)i1))),
-                   sclL3(b2, ld3(sc.tan + 3 * (size_t)i2)));
+    if (mf & MESH_HAS_TANGENTS)
+    {
+        const MeshRec   me = sc.meshes[ip->mesh];
+        const uint32_t* ix = sc.idx + 3 * (size_t)(me.idx_off + h.prim);
+        const float*    tv = sc.tan + 3 * (size_t)me.vtx_off;
+        tgo = add3(add3(sclL3(b0, ld3(tv + 3 * (size_t)ix[0])), sclL3(b1, ld3(tv + 3 * (size_t)ix[1]))),
+                   sclL3(b2, ld3(tv + 3 * (size_t)ix[2])));
+    }
     float M[12], I[12];
 #pragma unroll
     for (int k = 0; k < 12; ++k)
@@ -1000,7 +1002,7 @@ __global__ __launch_bounds__(256) void k_shade(SceneView sc, BatchTable bt, uint
                     const float4 hh = hb.h[i0];
                     sh_h[w]         = hh;
                     sh_d[w]         = qin.d[i0];
-                    cls[g] = __float_as_uint(hh.z) != CLPT_NO_HIT ? 1u + sc.mtl[sc.inst[__float_as_uint(hh.z)].material].type : 0u;
+                    cls[g] = __float_as_uint(hh.z) != CLPT_NO_HIT ? 1u + sc.inst[__float_as_uint(hh.z)].mtl_type : 0u;
                 }
             }
 #pragma unroll
@@ -1206,7 +1208,7 @@ __global__ __launch_bounds__(256, 2) void k_shade_guided(SceneView sc, BatchTabl
                 if (i0 < n)
                 {
                     const float4 hh = hb.h[i0];
-                    cls[g] = __float_as_uint(hh.z) != CLPT_NO_HIT ? 1u + sc.mtl[sc.inst[__float_as_uint(hh.z)].material].type : 0u;
+                    cls[g] = __float_as_uint(hh.z) != CLPT_NO_HIT ? 1u + sc.inst[__float_as_uint(hh.z)].mtl_type : 0u;
                 }
             }
 #pragma unroll
@@ -1826,7 +1828,32 @@ __global__ __launch_bounds__(256) void k_dome_cuts(uint32_t w, uint32_t h, const
     }
 }
 
-/* ------------------------------------------------------------ tree packing */
+/* ------------------------------------------------------------ scene packing */
+
+/* The shading records of one mesh, a thread per triangle. */
+__global__ __launch_bounds__(256) void k_shade_recs(MeshRec me, const uint32_t* __restrict__ idx, const float* __restrict__ pos,
+                                                    const float* __restrict__ nrm, const float* __restrict__ uv,
+                                                    ShadeRec* __restrict__ out)
+{
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= me.ntris)
+        return;
+    const size_t g = (size_t)me.idx_off + t;
+    ShadeRec     r{};
+    for (int k = 0; k < 3; ++k)
+    {
+        const size_t v = (size_t)idx[3 * g + k] + me.vtx_off;
+        for (int a = 0; a < 3; ++a)
+        {
+            r.p[k][a] = pos[3 * v + a];
+            r.n[k][a] = me.flags & MESH_HAS_NORMALS ? nrm[3 * v + a] : 0.0f;
+        }
+        for (int a = 0; a < 2; ++a)
+            r.uv[k][a] = me.flags & MESH_HAS_UVS ? uv[2 * v + a] : 0.0f;
+    }
+    out[g] = r;
+}
+
 
 /* One thread per BVH4 node: the packed form of its float boxes. */
 __global__ __launch_bounds__(256) void k_pack_nodes(const Node4* __restrict__ in, uint32_t n, Node4P* __restrict__ out)
@@ -2161,6 +2188,14 @@ hipError_t launch_srgb_batch(hipStream_t s, const float* in, uint32_t n, int dec
 hipError_t launch_texture_u8(hipStream_t s, const uchar4* in, uint32_t n, int srgb, float4* out)
 {
     hipLaunchKernelGGL(k_texture_u8, dim3(grid_for(n, 256, 4096)), dim3(256), 0, s, in, n, srgb, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_shade_recs(hipStream_t s, const MeshRec& me, const uint32_t* idx, const float* pos, const float* nrm,
+                             const float* uv, ShadeRec* out)
+{
+    if (me.ntris)
+        hipLaunchKernelGGL(k_shade_recs, dim3((me.ntris + 255u) / 256u), dim3(256), 0, s, me, idx, pos, nrm, uv, out);
     return hipGetLastError();
 }
 
