@@ -151,7 +151,7 @@ struct clhip_ctx
     std::vector<EmitterRec> emitters;
     int32_t                 dome_index = -1, dome_tex = -1;
     uint32_t                dome_w = 0, dome_h = 0;
-    DevBuf                  d_emitters, d_pcond, d_cdfcond, d_pv, d_cdfv, d_rowint, d_cutv, d_cutcond;
+    DevBuf                  d_emitters, d_domeq, d_pcond, d_cdfcond, d_pv, d_cdfv, d_rowint, d_cutv, d_cutcond;
 
     /* camera / parameters (the single-view film) */
     ViewRec      cam{};
@@ -291,11 +291,10 @@ SceneView scene_view(const clhip_ctx* c)
     s.dome_index = c->dome_index;
     if (c->dome_tex >= 0)
     {
-        s.dome_tex = c->textures[c->dome_tex].buf->as<const float4>();
+        s.dome_tex = c->d_domeq.as<const float4>();
         s.dome_w   = c->dome_w;
         s.dome_h   = c->dome_h;
     }
-    s.pcond     = c->d_pcond.as<const float>();
     s.cdfcond   = c->d_cdfcond.as<const float>();
     s.pv        = c->d_pv.as<const float>();
     s.cdfv      = c->d_cdfv.as<const float>();
@@ -1773,6 +1772,7 @@ int clhip_build_emitters(clhip_ctx* ctx, const clhip_emitter* emitters, uint32_t
         const size_t W   = (size_t)t.w + 1;
         CLHIP_CHECK(ctx, ctx->d_pcond.alloc(W * t.h * sizeof(float)));
         CLHIP_CHECK(ctx, ctx->d_cdfcond.alloc(W * t.h * sizeof(float)));
+        CLHIP_CHECK(ctx, ctx->d_domeq.alloc((size_t)t.w * t.h * sizeof(float4)));
         CLHIP_CHECK(ctx, ctx->d_pv.alloc(((size_t)t.h + 1) * sizeof(float)));
         CLHIP_CHECK(ctx, ctx->d_cdfv.alloc(((size_t)t.h + 1) * sizeof(float)));
         CLHIP_CHECK(ctx, ctx->d_rowint.alloc((size_t)t.h * sizeof(double)));
@@ -1782,7 +1782,7 @@ int clhip_build_emitters(clhip_ctx* ctx, const clhip_emitter* emitters, uint32_t
                                                   ctx->d_pcond.as<float>(), ctx->d_cdfcond.as<float>(),
                                                   ctx->d_pv.as<float>(), ctx->d_cdfv.as<float>(),
                                                   ctx->d_rowint.as<double>(), ctx->d_cutv.as<uint32_t>(),
-                                                  ctx->d_cutcond.as<uint32_t>()));
+                                                  ctx->d_cutcond.as<uint32_t>(), ctx->d_domeq.as<float4>()));
         CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     }
     return CLHIP_OK;

@@ -480,10 +480,18 @@ CLPT_D f3 bsdf_sample(const MaterialRec& m, f3 wo, float ux, float uy, float u_l
 
 /* ------------------------------------------------------------ textures */
 
-/* Exact bilinear RGBA32F fetch, wrap addressing, normalized coordinates:
- * the renderer's ImageTexture2D::eval2D (imagetex2d.h:34-37; sampler state
- * src/core/nodes/textures/imagetex2d.cpp:50-66). */
-CLPT_D float4 tex_eval(const float4* tex, uint32_t w, uint32_t h, float u, float v)
+/* The four texels and weights of an exact bilinear RGBA32F fetch with wrap
+ * addressing and normalized coordinates (ImageTexture2D::eval2D,
+ * imagetex2d.h:34-37; sampler state src/core/nodes/textures/
+ * imagetex2d.cpp:50-66). */
+struct TexQuad
+{
+    int    ix0, ix1, iy0, iy1;
+    float4 t00, t10, t01, t11;
+    float  w00, w10, w01, w11;
+};
+
+CLPT_D void tex_quad(const float4* tex, uint32_t w, uint32_t h, float u, float v, TexQuad& q)
 {
     const float uu = u - floorf(u);
     const float vv = v - floorf(v);
@@ -494,22 +502,33 @@ CLPT_D float4 tex_eval(const float4* tex, uint32_t w, uint32_t h, float u, float
     int         ix0 = (int)fx, iy0 = (int)fy;
     int         ix1 = ix0 + 1, iy1 = iy0 + 1;
     const int   W = (int)w, H = (int)h;
-    ix0 = ix0 < 0 ? ix0 + W : (ix0 >= W ? ix0 - W : ix0);
-    ix1 = ix1 < 0 ? ix1 + W : (ix1 >= W ? ix1 - W : ix1);
-    iy0 = iy0 < 0 ? iy0 + H : (iy0 >= H ? iy0 - H : iy0);
-    iy1 = iy1 < 0 ? iy1 + H : (iy1 >= H ? iy1 - H : iy1);
-    const float4 t00 = tex[(size_t)iy0 * W + ix0];
-    const float4 t10 = tex[(size_t)iy0 * W + ix1];
-    const float4 t01 = tex[(size_t)iy1 * W + ix0];
-    const float4 t11 = tex[(size_t)iy1 * W + ix1];
-    const float  w00 = (1.0f - ax) * (1.0f - ay);
-    const float  w10 = ax * (1.0f - ay);
-    const float  w01 = (1.0f - ax) * ay;
-    const float  w11 = ax * ay;
-    return make_float4(w00 * t00.x + w10 * t10.x + w01 * t01.x + w11 * t11.x,
-                       w00 * t00.y + w10 * t10.y + w01 * t01.y + w11 * t11.y,
-                       w00 * t00.z + w10 * t10.z + w01 * t01.z + w11 * t11.z,
-                       w00 * t00.w + w10 * t10.w + w01 * t01.w + w11 * t11.w);
+    q.ix0 = ix0 < 0 ? ix0 + W : (ix0 >= W ? ix0 - W : ix0);
+    q.ix1 = ix1 < 0 ? ix1 + W : (ix1 >= W ? ix1 - W : ix1);
+    q.iy0 = iy0 < 0 ? iy0 + H : (iy0 >= H ? iy0 - H : iy0);
+    q.iy1 = iy1 < 0 ? iy1 + H : (iy1 >= H ? iy1 - H : iy1);
+    q.t00 = tex[(size_t)q.iy0 * W + q.ix0];
+    q.t10 = tex[(size_t)q.iy0 * W + q.ix1];
+    q.t01 = tex[(size_t)q.iy1 * W + q.ix0];
+    q.t11 = tex[(size_t)q.iy1 * W + q.ix1];
+    q.w00 = (1.0f - ax) * (1.0f - ay);
+    q.w10 = ax * (1.0f - ay);
+    q.w01 = (1.0f - ax) * ay;
+    q.w11 = ax * ay;
+}
+
+CLPT_D f3 tex_quad_rgb(const TexQuad& q)
+{
+    return f3{q.w00 * q.t00.x + q.w10 * q.t10.x + q.w01 * q.t01.x + q.w11 * q.t11.x,
+              q.w00 * q.t00.y + q.w10 * q.t10.y + q.w01 * q.t01.y + q.w11 * q.t11.y,
+              q.w00 * q.t00.z + q.w10 * q.t10.z + q.w01 * q.t01.z + q.w11 * q.t11.z};
+}
+
+/* rgb of a texture lookup (no caller uses a texture's alpha) */
+CLPT_D f3 tex_eval(const float4* tex, uint32_t w, uint32_t h, float u, float v)
+{
+    TexQuad q;
+    tex_quad(tex, w, h, u, v, q);
+    return tex_quad_rgb(q);
 }
 
 /* ------------------------------------------------------------ emitters */
@@ -539,9 +558,10 @@ CLPT_D uint32_t upper_bound_cut(const float* a, const uint32_t* cut, float value
     return upper_bound_f(a, cut[k], cut[k + 1], value);
 }
 
-/* cut: the CDF's cut points, or NULL for a search of the whole CDF */
-CLPT_D float sample1d(const float* f, const float* cdf, uint32_t N, float c, float u, uint32_t cdf_off, float* pdf,
-                      uint32_t* off, const uint32_t* cut)
+/* f: the N function values, fstride floats apart; cut: the CDF's cut points,
+ * or NULL for a search of the whole CDF */
+CLPT_D float sample1d(const float* f, uint32_t fstride, const float* cdf, uint32_t N, float c, float u, uint32_t cdf_off,
+                      float* pdf, uint32_t* off, const uint32_t* cut)
 {
     if (c == 0.0f)
         return 0.0f;
@@ -551,11 +571,11 @@ CLPT_D float sample1d(const float* f, const float* cdf, uint32_t N, float c, flo
         o = cdf_off;
     if (o > cdf_off + N - 1)
         o = cdf_off + N - 1;
-    *pdf     = f[o] / c;
     float du = u - cdf[o];
     if (cdf[o + 1] - cdf[o] != 0.0f)
         du /= cdf[o + 1] - cdf[o];
     o -= cdf_off;
+    *pdf = f[(size_t)o * fstride] / c;
     *off = o;
     return ((float)o + du) / (float)N;
 }
@@ -566,15 +586,20 @@ CLPT_D void sample2d(const SceneView& sc, float ux, float uy, float* su, float* 
     const uint32_t nu = sc.dome_w, nv = sc.dome_h;
     float          pu = 0.0f, pvv = 0.0f;
     uint32_t       off = 0;
-    *sv                = sample1d(sc.pv, sc.cdfv, nv, sc.pv[nv], uy, 0, &pvv, &off, sc.cutv);
-    const float cv     = sc.pcond[(size_t)off * (nu + 1) + nu];
-    *su = sample1d(sc.pcond, sc.cdfcond, nu, cv, ux, off * (nu + 1), &pu, &off,
+    *sv                = sample1d(sc.pv, 1u, sc.cdfv, nv, sc.pv[nv], uy, 0, &pvv, &off, sc.cutv);
+    /* the row's integral (pcond's last entry, which pv holds too) and its
+     * function values (the texels' w, in the lines the lookup at the sampled
+     * point reads) */
+    const float cv = sc.pv[off];
+    *su = sample1d(&sc.dome_tex[(size_t)off * nu].w, 4u, sc.cdfcond, nu, cv, ux, off * (nu + 1), &pu, &off,
                    sc.cutcond ? sc.cutcond + (size_t)off * (CLPT_CUTS + 1u) : nullptr);
     *pdf               = pu * pvv;
 }
 
-/* Distribution2D::pdf2D: hdridome.h:125-135 */
-CLPT_D float pdf2d(const SceneView& sc, float u, float v)
+/* Distribution2D::pdf2D (hdridome.h:125-135) at (u, v), whose texel is one
+ * of the four that the lookup there read: x = u w - 0.5 floors to the texel
+ * of u w or the one before it.  (Any other index, as of a NaN, is read.) */
+CLPT_D float pdf2d(const SceneView& sc, float u, float v, const TexQuad& q)
 {
     if (u < 0.0f || v < 0.0f)
         return 0.0f;
@@ -584,7 +609,13 @@ CLPT_D float pdf2d(const SceneView& sc, float u, float v)
         iu = sc.dome_w - 1;
     if (iv > sc.dome_h - 1)
         iv = sc.dome_h - 1;
-    return sc.pcond[(size_t)iv * (sc.dome_w + 1) + iu] / sc.pv[sc.dome_h];
+    const bool x0 = (int)iu == q.ix0, y0 = (int)iv == q.iy0;
+    float      f;
+    if ((x0 || (int)iu == q.ix1) && (y0 || (int)iv == q.iy1))
+        f = x0 ? (y0 ? q.t00.w : q.t01.w) : (y0 ? q.t10.w : q.t11.w);
+    else
+        f = sc.dome_tex[(size_t)iv * sc.dome_w + iu].w;
+    return f / sc.pv[sc.dome_h];
 }
 
 /* cos(theta) of a direction for acos: clamped to [-1, 1], since a unit
@@ -592,27 +623,26 @@ CLPT_D float pdf2d(const SceneView& sc, float u, float v)
  * (the reference passes dir.y unclamped and gets NaN there). */
 CLPT_D float dome_cos_theta(f3 dir) { return fminf(1.0f, fmaxf(-1.0f, dir.y)); }
 
-/* HDRIDome::evalEnvironment + directionToUVCoords: hdridome.h:291-297, 472-476 */
-CLPT_D f3 dome_le(const SceneView& sc, f3 dir)
-{
-    const float  u = clpt_atan2f(dir.x, dir.z) * -CLPT_INV_PI_F * 0.5f + 0.5f;
-    const float  v = clpt_acosf(dome_cos_theta(dir)) * CLPT_INV_PI_F;
-    const float4 c = tex_eval(sc.dome_tex, sc.dome_w, sc.dome_h, u, v);
-    return f3{c.x, c.y, c.z};
-}
-
-/* HDRIDome::pdfDirect: hdridome.h:248-279 */
-CLPT_D float dome_pdf(const SceneView& sc, f3 dir)
+/* HDRIDome::evalEnvironment + directionToUVCoords (hdridome.h:291-297,
+ * 472-476) and, where pdf is wanted, HDRIDome::pdfDirect (:248-279) of the
+ * same direction: one texel quad serves both, its w holding the sampling
+ * function (a lookup of its own in the table cost one more cache line per
+ * escaped ray). */
+CLPT_D f3 dome_le(const SceneView& sc, f3 dir, float* pdf = nullptr)
 {
     const float phi   = clpt_atan2f(dir.x, dir.z);
     const float theta = clpt_acosf(dome_cos_theta(dir));
-    float       st, ct;
-    clpt_sincosf(theta, &st, &ct);
-    if (st == 0.0f)
-        return 0.0f;
-    const float u = phi * -CLPT_INV_PI_F * 0.5f + 0.5f;
-    const float v = theta * CLPT_INV_PI_F;
-    return pdf2d(sc, u, v) / (2.0f * CLPT_PI_F * CLPT_PI_F * st);
+    const float u     = phi * -CLPT_INV_PI_F * 0.5f + 0.5f;
+    const float v     = theta * CLPT_INV_PI_F;
+    TexQuad     q;
+    tex_quad(sc.dome_tex, sc.dome_w, sc.dome_h, u, v, q);
+    if (pdf)
+    {
+        float st, ct;
+        clpt_sincosf(theta, &st, &ct);
+        *pdf = st == 0.0f ? 0.0f : pdf2d(sc, u, v, q) / (2.0f * CLPT_PI_F * CLPT_PI_F * st);
+    }
+    return tex_quad_rgb(q);
 }
 
 /* HDRIDome::sampleDirect: hdridome.h:186-228 */
@@ -632,8 +662,7 @@ CLPT_D f3 dome_sample(const SceneView& sc, float ux, float uy, f3* dir, float* p
     }
     *dir           = f3{st * sp, ct, st * cp};
     *pdf           = p / (2.0f * CLPT_PI_F * CLPT_PI_F * st);
-    const float4 c = tex_eval(sc.dome_tex, sc.dome_w, sc.dome_h, su, sv);
-    return f3{c.x, c.y, c.z};
+    return tex_eval(sc.dome_tex, sc.dome_w, sc.dome_h, su, sv);
 }
 
 /* DirectionalEmitter::sampleDirect: directional.h:30-56 */

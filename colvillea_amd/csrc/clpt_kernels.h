@@ -47,7 +47,7 @@ hipError_t launch_shade_recs(hipStream_t s, const MeshRec& me, const uint32_t* i
 /* The traversal form of n BVH4 nodes. */
 hipError_t launch_pack_nodes(hipStream_t s, const Node4* in, uint32_t n, Node4P* out);
 hipError_t launch_dome_tables(hipStream_t s, const float4* tex, uint32_t w, uint32_t h, float* pcond, float* cdfcond,
-                              float* pv, float* cdfv, double* rowint, uint32_t* cutv, uint32_t* cutcond);
+                              float* pv, float* cdfv, double* rowint, uint32_t* cutv, uint32_t* cutcond, float4* packed);
 hipError_t launch_rng_batch(hipStream_t s, const uint4* seeds, uint32_t n, uint32_t ndraws, uint32_t* ou, float* of);
 hipError_t launch_camera_batch(hipStream_t s, const ViewRec& fr, const uint2* ps, uint32_t n, float4* out);
 hipError_t launch_bsdf_batch(hipStream_t s, const SceneView& sc, const uint32_t* mtl, const float* wi3,

@@ -176,9 +176,8 @@ struct SceneView
     const EmitterRec*  emitters;
     uint32_t           nemitters;
     int32_t            dome_index;
-    const float4*      dome_tex;
+    const float4*      dome_tex; /* rgb and, in w, the texel's value of the sampling function (pcond) */
     uint32_t           dome_w, dome_h;
-    const float*       pcond;
     const float*       cdfcond;
     const float*       pv;
     const float*       cdfv;

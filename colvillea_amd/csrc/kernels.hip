@@ -651,7 +651,7 @@ __device__ __forceinline__ void material_at(const SceneView& sc, MaterialRec& m,
     if (m.tex_r)
     {
         const TexRec t = sc.tex[m.tex_r - 1u];
-        const float4 c = tex_eval(t.data, t.w, t.h, si.u, si.v);
+        const f3     c = tex_eval(t.data, t.w, t.h, si.u, si.v);
         m.r[0]         = c.x;
         m.r[1]         = c.y;
         m.r[2]         = c.z;
@@ -665,7 +665,7 @@ __device__ __forceinline__ void material_at(const SceneView& sc, MaterialRec& m,
     if (m.tex_n)
     {
         const TexRec t  = sc.tex[m.tex_n - 1u];
-        const float4 c  = tex_eval(t.data, t.w, t.h, si.u, si.v);
+        const f3     c  = tex_eval(t.data, t.w, t.h, si.u, si.v);
         const f3     nt = f3{c.x * 2.0f - 1.0f, c.y * 2.0f - 1.0f, c.z * 2.0f - 1.0f};
         if (dot3(nt, nt) > 0.0f)
         {
@@ -1052,12 +1052,13 @@ __global__ __launch_bounds__(256) void k_shade(SceneView sc, BatchTable bt, uint
         f3 esc{0.0f, 0.0f, 0.0f};
         if (!hit && dome)
         {
-            const f3 le = dome_le(sc, dir);
             if (depth == 1)
-                esc = le;
+                esc = dome_le(sc, dir);
             else
             {
-                const float lp = dome_pdf(sc, dir) / nl;
+                float       lp;
+                const f3    le = dome_le(sc, dir, &lp);
+                lp /= nl;
                 const float w  = T4.w / (T4.w + lp);
                 esc            = mul3(T, scl3(le, w));
             }
@@ -1295,12 +1296,13 @@ __global__ __launch_bounds__(256, 2) void k_shade_guided(SceneView sc, BatchTabl
         f3 esc{0.0f, 0.0f, 0.0f};
         if (active && !hit && dome)
         {
-            const f3 le = dome_le(sc, dir);
             if (depth == 1)
-                esc = le;
+                esc = dome_le(sc, dir);
             else
             {
-                const float lp = dome_pdf(sc, dir) / nl;
+                float       lp;
+                const f3    le = dome_le(sc, dir, &lp);
+                lp /= nl;
                 const float w  = T4.w / (T4.w + lp);
                 esc            = mul3(T, scl3(le, w));
             }
@@ -1773,6 +1775,19 @@ __global__ __launch_bounds__(256) void k_dome_rows(uint32_t w, uint32_t h, float
     }
 }
 
+/* The dome's texels as shading reads them: rgb of the texture, the sampling
+ * function's value in w. */
+__global__ __launch_bounds__(256) void k_dome_pack(const float4* __restrict__ tex, uint32_t w, uint32_t h,
+                                                   const float* __restrict__ pcond, float4* __restrict__ out)
+{
+    const uint32_t total = w * h;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < total; i += gridDim.x * blockDim.x)
+    {
+        const float4 c = tex[i];
+        out[i]         = make_float4(c.x, c.y, c.z, pcond[(size_t)(i / w) * (w + 1) + i % w]);
+    }
+}
+
 /* preprocessPV (hdridome.h:387-432) in float64: one block. */
 __global__ __launch_bounds__(256) void k_dome_marginal(uint32_t h, float* pv, float* cdfv, const double* rowint)
 {
@@ -1941,11 +1956,10 @@ __global__ void k_dome_eval_batch(SceneView sc, const float* dir3, uint32_t n, f
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
     {
         const f3 d  = ld3(dir3 + 3 * (size_t)i);
-        const f3 le = dome_le(sc, d);
+        const f3 le = dome_le(sc, d, pdf + i);
         le3[3 * i]     = le.x;
         le3[3 * i + 1] = le.y;
         le3[3 * i + 2] = le.z;
-        pdf[i]         = dome_pdf(sc, d);
     }
 }
 
@@ -2207,10 +2221,11 @@ hipError_t launch_pack_nodes(hipStream_t s, const Node4* in, uint32_t n, Node4P*
 }
 
 hipError_t launch_dome_tables(hipStream_t s, const float4* tex, uint32_t w, uint32_t h, float* pcond, float* cdfcond,
-                              float* pv, float* cdfv, double* rowint, uint32_t* cutv, uint32_t* cutcond)
+                              float* pv, float* cdfv, double* rowint, uint32_t* cutv, uint32_t* cutcond, float4* packed)
 {
     hipLaunchKernelGGL(k_dome_prefilter, dim3(grid_for((uint64_t)w * h, 256, 8192)), dim3(256), 0, s, tex, w, h, pcond);
     hipLaunchKernelGGL(k_dome_rows, dim3(h), dim3(256), 0, s, w, h, pcond, cdfcond, pv, rowint);
+    hipLaunchKernelGGL(k_dome_pack, dim3(grid_for((uint64_t)w * h, 256, 8192)), dim3(256), 0, s, tex, w, h, pcond, packed);
     hipLaunchKernelGGL(k_dome_marginal, dim3(1), dim3(256), 0, s, h, pv, cdfv, rowint);
     hipLaunchKernelGGL(k_dome_cuts, dim3(h + 1), dim3(256), 0, s, w, h, cdfcond, cdfv, cutv, cutcond);
     return hipGetLastError();
