@@ -7,6 +7,7 @@
 #include "bvh_build.h"
 #include "clpt_guide.h"
 #include "clpt_kernels.h"
+#include "host_copy.h"
 
 #include <hip/hip_runtime.h>
 
@@ -159,6 +160,7 @@ struct clhip_ctx
     clhip_params params{5u, 0u, 0u, 0u};
 
     /* render state */
+    std::unique_ptr<clpt::HostCopier> copier; /* large copies to and from the caller's memory */
     DevBuf   d_accum, d_out;
     DevBuf   d_q[2][3], d_hit, d_sq[3], d_pacc, d_gstack, d_bc, d_tot, d_ctr;
     size_t   qcap = 0;
@@ -177,7 +179,7 @@ struct clhip_ctx
     uint64_t              graph_clock = 0;
 
     /* multi-view film */
-    DevBuf                d_vaccum;
+    DevBuf                d_vaccum, d_vout;
     std::vector<ViewRec>  vviews;
     std::vector<uint32_t> vspp, vlast_batch;
     std::vector<hipEvent_t> batch_events;
@@ -188,6 +190,7 @@ struct clhip_ctx
     clhip_guide guide{};
     bool        guide_ready = false;
     DevBuf      g_params, g_m1, g_m2, g_W, g_WT, g_img, g_gc, g_img8, g_scl;
+    DevBuf      g_raw, g_gradout; /* clhip_guide_train: the caller's samples, the gradient */
     DevBuf      g_X, g_act[4], g_out, g_grad[5], g_loss, g_wpart, g_spart, g_amaxp, g_partial, g_samples;
     uint32_t    g_partcap = 0; /* blocks the per-block gradient buffers hold */
     uint32_t    g_N = 0;
@@ -1155,6 +1158,7 @@ int clhip_create(uint32_t width, uint32_t height, uint32_t integrator_type, clhi
     c->cam.width  = width;
     c->cam.height = height;
     c->cam.npix   = width * height;
+    c->copier = std::make_unique<clpt::HostCopier>(c->device);
     *out         = c.release();
     return CLHIP_OK;
 }
@@ -2084,9 +2088,8 @@ int clhip_view_sums(clhip_ctx* ctx, uint32_t view, double* rgb, size_t bytes)
     const ViewRec& v = ctx->vviews[view];
     if (bytes < (size_t)v.npix * 3 * sizeof(double))
         return fail(ctx, CLHIP_E_INVALID, "clhip_view_sums: buffer too small");
-    CLHIP_CHECK(ctx, hipMemcpyAsync(rgb, ctx->d_vaccum.as<double>() + 3 * (size_t)v.film_offset,
-                                    (size_t)v.npix * 3 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    CLHIP_CHECK(ctx, ctx->copier->to_host(ctx->stream, rgb, ctx->d_vaccum.as<double>() + 3 * (size_t)v.film_offset,
+                                          (size_t)v.npix * 3 * sizeof(double)));
     return CLHIP_OK;
 }
 
@@ -2099,12 +2102,10 @@ int clhip_view_readback(clhip_ctx* ctx, uint32_t view, float* rgba, size_t bytes
     const ViewRec& v = ctx->vviews[view];
     if (bytes < (size_t)v.npix * 16)
         return fail(ctx, CLHIP_E_INVALID, "clhip_view_readback: buffer too small");
-    DevBuf out;
-    CLHIP_CHECK(ctx, out.alloc((size_t)v.npix * 16));
+    CLHIP_CHECK(ctx, ctx->d_vout.alloc((size_t)v.npix * 16)); /* nothing in flight reads it: readbacks wait */
     CLHIP_CHECK(ctx, clpt::launch_resolve(ctx->stream, ctx->d_vaccum.as<double>() + 3 * (size_t)v.film_offset, v.npix,
-                                          ctx->vspp[view], 0, out.as<float4>()));
-    CLHIP_CHECK(ctx, hipMemcpyAsync(rgba, out.p, (size_t)v.npix * 16, hipMemcpyDeviceToHost, ctx->stream));
-    CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+                                          ctx->vspp[view], 0, ctx->d_vout.as<float4>()));
+    CLHIP_CHECK(ctx, ctx->copier->to_host(ctx->stream, rgba, ctx->d_vout.p, (size_t)v.npix * 16));
     return CLHIP_OK;
 }
 
@@ -2151,8 +2152,7 @@ static int readback_film(clhip_ctx* ctx, float* rgba, size_t bytes, int srgb, co
     }
     CLHIP_CHECK(ctx, clpt::launch_resolve(ctx->stream, ctx->d_accum.as<double>(), (uint32_t)npix, ctx->spp, srgb,
                                           ctx->d_out.as<float4>()));
-    CLHIP_CHECK(ctx, hipMemcpyAsync(rgba, ctx->d_out.p, npix * 16, hipMemcpyDeviceToHost, ctx->stream));
-    CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    CLHIP_CHECK(ctx, ctx->copier->to_host(ctx->stream, rgba, ctx->d_out.p, npix * 16));
     return CLHIP_OK;
 }
 
@@ -2190,8 +2190,7 @@ int clhip_readback_sums(clhip_ctx* ctx, double* rgb, size_t bytes)
         std::memset(rgb, 0, npix * 3 * sizeof(double));
         return CLHIP_OK;
     }
-    CLHIP_CHECK(ctx, hipMemcpyAsync(rgb, ctx->d_accum.p, npix * 3 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    CLHIP_CHECK(ctx, ctx->copier->to_host(ctx->stream, rgb, ctx->d_accum.p, npix * 3 * sizeof(double)));
     return CLHIP_OK;
 }
 
@@ -2586,8 +2585,7 @@ int clhip_guide_get_weights(clhip_ctx* ctx, float* w, uint32_t n)
         return fail(ctx, CLHIP_E_INVALID, "clhip_guide_get_weights: need %d floats", CLPT_G_PARAMS);
     if (!ctx->guide_ready)
         return fail(ctx, CLHIP_E_STATE, "no weights: call clhip_guide_reset or clhip_set_guide first");
-    CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    CLHIP_CHECK(ctx, hipMemcpy(w, ctx->g_params.p, CLPT_G_PARAMS * sizeof(float), hipMemcpyDeviceToHost));
+    CLHIP_CHECK(ctx, ctx->copier->to_host(ctx->stream, w, ctx->g_params.p, CLPT_G_PARAMS * sizeof(float)));
     return CLHIP_OK;
 }
 
@@ -2772,34 +2770,27 @@ int clhip_guide_train(clhip_ctx* ctx, const float* s13, uint32_t n, float* grad,
     int            rc = guide_train_buffers(ctx, N);
     if (rc)
         return rc;
-    std::vector<GuideSample> hs(n);
-    for (uint32_t i = 0; i < n; ++i)
-    {
-        const float* x = s13 + 13 * (size_t)i;
-        hs[i].a        = make_float4(x[0], x[1], x[2], x[3]);
-        hs[i].b        = make_float4(x[4], x[5], x[6], x[7]);
-        hs[i].c        = make_float4(x[8], x[9], x[10], x[11]);
-        hs[i].d        = make_float4(x[12], 0.0f, 0.0f, 0.0f);
-    }
-    CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    if (n)
-        CLHIP_CHECK(ctx, hipMemcpy(ctx->g_samples.p, hs.data(), n * sizeof(GuideSample), hipMemcpyHostToDevice));
-    CLHIP_CHECK(ctx, hipMemcpy(ctx->g_gc.p, &n, sizeof(uint32_t), hipMemcpyHostToDevice)); /* GuideCounters::count */
-    Tmp g;
-    if (grad)
-        CLHIP_CHECK(ctx, g.zeros(CLPT_G_PARAMS * sizeof(float)));
+    if ((size_t)n * 13 * sizeof(float) > ctx->g_raw.bytes)
+        CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream)); /* about to move */
+    CLHIP_CHECK(ctx, ctx->g_raw.alloc((size_t)n * 13 * sizeof(float)));
+    CLHIP_CHECK(ctx, ctx->g_gradout.alloc(CLPT_G_PARAMS * sizeof(float)));
+    CLHIP_CHECK(ctx, ctx->copier->from_host(ctx->stream, ctx->g_raw.p, s13, (size_t)n * 13 * sizeof(float)));
+    CLHIP_CHECK(ctx, clpt::launch_guide_samples(ctx->stream, ctx->g_raw.as<const float>(), n, ctx->g_samples.as<GuideSample>(),
+                                                ctx->g_gc.as<GuideCounters>()));
+    if (grad) /* a step without samples leaves it unwritten */
+        CLHIP_CHECK(ctx, hipMemsetAsync(ctx->g_gradout.p, 0, CLPT_G_PARAMS * sizeof(float), ctx->stream));
     CLHIP_CHECK(ctx, clpt::launch_guide_train(ctx->stream, guide_bufs(ctx), N,
                                               ctx->guide.learning_rate > 0.0f ? ctx->guide.learning_rate : 1e-3f,
-                                              grad ? g.b.as<float>() : nullptr, 0u, 1u));
-    CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+                                              grad ? ctx->g_gradout.as<float>() : nullptr, 0u, 1u));
     if (grad)
-        CLHIP_CHECK(ctx, g.to_host(grad, CLPT_G_PARAMS));
+        CLHIP_CHECK(ctx, ctx->copier->to_host(ctx->stream, grad, ctx->g_gradout.p, CLPT_G_PARAMS * sizeof(float)));
     if (loss)
     {
         GuideCounters gc;
-        CLHIP_CHECK(ctx, hipMemcpy(&gc, ctx->g_gc.p, sizeof(gc), hipMemcpyDeviceToHost));
+        CLHIP_CHECK(ctx, ctx->copier->to_host(ctx->stream, &gc, ctx->g_gc.p, sizeof(gc)));
         *loss = gc.loss;
     }
+    CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     return CLHIP_OK;
 }
 

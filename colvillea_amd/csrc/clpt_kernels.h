@@ -106,6 +106,8 @@ hipError_t launch_guide_mixture_batch(hipStream_t s, const float* out40, const f
                                       float* pdf, float* smp3, float* smp_pdf);
 hipError_t launch_guide_query_batch(hipStream_t s, const float lo[3], const float inv_ext[3], const float* p3,
                                     const float* n3, const float* wo3, uint32_t n, float* q9);
+/* n given samples of 13 floats as training samples, and their count */
+hipError_t launch_guide_samples(hipStream_t s, const float* s13, uint32_t n, GuideSample* out, GuideCounters* gc);
 hipError_t launch_guide_infer(hipStream_t s, const __bf16* img, const uint8_t* img8, const float* scl, const float* q9,
                               uint32_t n, float* out40, uint32_t blocks);
 hipError_t launch_guide_pack_fp8(hipStream_t s, const float* params, const GuideCounters* gc, uint8_t* img8,

@@ -1224,10 +1224,36 @@ __global__ __launch_bounds__(256) void k_guide_gather_write(const float4* V, con
     });
 }
 
+/* Given samples (13 floats each: query, direction, weight) as GuideSample
+ * records, and their count. */
+__global__ __launch_bounds__(256) void k_guide_samples(const float* __restrict__ s13, uint32_t n, GuideSample* __restrict__ out,
+                                                       GuideCounters* gc)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0u)
+        gc->count = n;
+    if (i >= n)
+        return;
+    const float* x = s13 + 13 * (size_t)i;
+    GuideSample  g;
+    g.a    = make_float4(x[0], x[1], x[2], x[3]);
+    g.b    = make_float4(x[4], x[5], x[6], x[7]);
+    g.c    = make_float4(x[8], x[9], x[10], x[11]);
+    g.d    = make_float4(x[12], 0.0f, 0.0f, 0.0f);
+    out[i] = g;
+}
+
 /* ------------------------------------------------------------ launchers */
 
 namespace clpt
 {
+hipError_t launch_guide_samples(hipStream_t s, const float* s13, uint32_t n, GuideSample* out, GuideCounters* gc)
+{
+    hipLaunchKernelGGL(k_guide_samples, dim3(std::max(1u, (n + 255u) / 256u)), dim3(256), 0, s, s13, n, out, gc);
+    return hipGetLastError();
+}
+
+
 hipError_t launch_guide_infer(hipStream_t s, const __bf16* img, const uint8_t* img8, const float* scl, const float* q9,
                               uint32_t n, float* out40, uint32_t blocks)
 {

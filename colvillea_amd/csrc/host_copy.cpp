@@ -1,0 +1,194 @@
+/* host_copy.cpp -- see host_copy.h. */
+#include "host_copy.h"
+
+#include <algorithm>
+#include <cstring>
+
+namespace clpt
+{
+HostCopier::~HostCopier()
+{
+    {
+        std::lock_guard<std::mutex> l(mu_);
+        stop_ = true;
+    }
+    wake_.notify_all();
+    for (std::thread& t : threads_)
+        t.join();
+    if (up_pending_)
+        (void)hipEventSynchronize(up_);
+    for (hipEvent_t e : ev_)
+        if (e)
+            (void)hipEventDestroy(e);
+    if (up_)
+        (void)hipEventDestroy(up_);
+    if (stage_)
+        (void)hipHostFree(stage_);
+}
+
+hipError_t HostCopier::reserve(size_t bytes)
+{
+    /* an upload may still be reading the staging */
+    if (up_pending_)
+    {
+        const hipError_t e = hipEventSynchronize(up_);
+        if (e != hipSuccess)
+            return e;
+        up_pending_ = false;
+    }
+    const size_t need = std::min(kStage, std::max<size_t>((bytes + kPiece - 1) / kPiece * kPiece, kPiece));
+    if (need > cap_)
+    {
+        if (stage_)
+            (void)hipHostFree(stage_);
+        stage_       = nullptr;
+        cap_         = 0;
+        void*      p = nullptr;
+        hipError_t e = hipHostMalloc(&p, need, hipHostMallocDefault);
+        if (e != hipSuccess)
+            return e;
+        stage_ = static_cast<char*>(p);
+        cap_   = need;
+    }
+    for (size_t k = 0; k < need / kPiece; ++k)
+        if (!ev_[k])
+        {
+            const hipError_t e = hipEventCreateWithFlags(&ev_[k], hipEventDisableTiming);
+            if (e != hipSuccess)
+                return e;
+        }
+    if (!up_)
+    {
+        const hipError_t e = hipEventCreateWithFlags(&up_, hipEventDisableTiming);
+        if (e != hipSuccess)
+            return e;
+    }
+    if (bytes > 2 * kPiece && threads_.empty())
+        try
+        {
+            for (unsigned k = 1; k < kThreads; ++k)
+                threads_.emplace_back([this] { work(); });
+        }
+        catch (...)
+        {
+            /* as many as could be started; the caller's thread does the rest */
+        }
+    return hipSuccess;
+}
+
+void HostCopier::work()
+{
+    (void)hipSetDevice(device_);
+    uint64_t seen = 0;
+    for (;;)
+    {
+        const std::function<void(size_t)>* job = nullptr;
+        size_t                             n   = 0;
+        {
+            std::unique_lock<std::mutex> l(mu_);
+            wake_.wait(l, [&] { return stop_ || (job_ && round_ != seen); });
+            if (stop_)
+                return;
+            seen = round_;
+            job  = job_;
+            n    = njobs_;
+            ++busy_;
+        }
+        for (size_t k = next_++; k < n; k = next_++)
+            (*job)(k);
+        {
+            std::lock_guard<std::mutex> l(mu_);
+            --busy_;
+        }
+        idle_.notify_one();
+    }
+}
+
+void HostCopier::run(size_t n, const std::function<void(size_t)>& job)
+{
+    if (n < 3 || threads_.empty())
+    {
+        for (size_t k = 0; k < n; ++k)
+            job(k);
+        return;
+    }
+    {
+        std::lock_guard<std::mutex> l(mu_);
+        job_   = &job;
+        njobs_ = n;
+        next_  = 0;
+        ++round_;
+    }
+    wake_.notify_all();
+    for (size_t k = next_++; k < n; k = next_++)
+        job(k);
+    /* no thread takes the job up any more, and those that did are done */
+    std::unique_lock<std::mutex> l(mu_);
+    job_ = nullptr;
+    idle_.wait(l, [&] { return busy_ == 0; });
+}
+
+hipError_t HostCopier::to_host(hipStream_t s, void* dst, const void* dev, size_t bytes)
+{
+    if (!bytes)
+        return hipStreamSynchronize(s);
+    hipError_t e = reserve(bytes);
+    if (e != hipSuccess)
+        return e;
+    char*       out = static_cast<char*>(dst);
+    const char* in  = static_cast<const char*>(dev);
+    for (size_t at = 0; at < bytes; at += cap_)
+    {
+        const size_t part = std::min(cap_, bytes - at), n = (part + kPiece - 1) / kPiece;
+        for (size_t k = 0; k < n; ++k)
+        {
+            const size_t len = std::min(kPiece, part - k * kPiece);
+            e = hipMemcpyAsync(stage_ + k * kPiece, in + at + k * kPiece, len, hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess)
+                e = hipEventRecord(ev_[k], s);
+            if (e != hipSuccess)
+            {
+                (void)hipStreamSynchronize(s); /* the pieces queued so far */
+                return e;
+            }
+        }
+        std::atomic<int> bad{(int)hipSuccess};
+        run(n, [&](size_t k) {
+            const hipError_t w = hipEventSynchronize(ev_[k]);
+            if (w != hipSuccess)
+                bad = (int)w;
+            else
+                std::memcpy(out + at + k * kPiece, stage_ + k * kPiece, std::min(kPiece, part - k * kPiece));
+        });
+        if (bad != (int)hipSuccess)
+            return (hipError_t)bad.load();
+    }
+    return hipSuccess;
+}
+
+hipError_t HostCopier::from_host(hipStream_t s, void* dev, const void* src, size_t bytes)
+{
+    const char* in  = static_cast<const char*>(src);
+    char*       out = static_cast<char*>(dev);
+    for (size_t at = 0; at < bytes; at += cap_)
+    {
+        hipError_t e = reserve(bytes);
+        if (e != hipSuccess)
+            return e;
+        const size_t part = std::min(cap_, bytes - at);
+        run((part + kPiece - 1) / kPiece, [&](size_t k) {
+            std::memcpy(stage_ + k * kPiece, in + at + k * kPiece, std::min(kPiece, part - k * kPiece));
+        });
+        e = hipMemcpyAsync(out + at, stage_, part, hipMemcpyHostToDevice, s);
+        if (e == hipSuccess)
+            e = hipEventRecord(up_, s);
+        if (e != hipSuccess)
+        {
+            (void)hipStreamSynchronize(s);
+            return e;
+        }
+        up_pending_ = true;
+    }
+    return hipSuccess;
+}
+} // namespace clpt
