@@ -626,6 +626,11 @@ bool use_graph(const clhip_ctx* c) { return !c->timing && c->launch.graph != 2u;
  * and shading of the first bounces see more compact groups of rays). */
 uint32_t launch_tile(const clhip_ctx* c) { return c->launch.tile ? c->launch.tile : 16u; }
 
+/* Pixels whose samples are traced together.  Batches that record training
+ * paths keep the film's pixels together instead, sample by sample: the
+ * recorded paths are drawn by path number. */
+uint32_t pixel_group(const clhip_ctx* c) { return guide_recording(c) ? (1u << 30) : CLPT_PIXEL_GROUP; }
+
 /* WavefrontDirectLightingIntegrator (direct.cpp:84-201,
  * raygeneration.cu:139-282): at the first hit one light sample and one BSDF
  * sample, MIS-weighted against each other, the BSDF ray counting only if it
@@ -717,8 +722,7 @@ BatchArgs batch_args(clhip_ctx* c, double* accum, uint32_t max_depth, bool singl
     BatchArgs a{};
     a.sc = scene_view(c);
     a.bt = BatchTable{c->d_views.as<const ViewRec>(), c->d_batches.as<const BatchRec>(),
-                      c->d_entries.as<const BatchEntry>(), c->d_cursor.as<uint32_t>(),
-                      launch_tile(c)};
+                      c->d_entries.as<const BatchEntry>(), c->d_cursor.as<uint32_t>(), pixel_group(c), launch_tile(c)};
     for (int k = 0; k < 2; ++k)
     {
         a.q[k].o     = c->d_q[k][0].as<float4>();
@@ -1918,7 +1922,7 @@ int clhip_render(clhip_ctx* ctx, uint32_t spp)
     {
         const uint32_t nb = std::min(spb, spp - done);
         batches.push_back(BatchRec{(uint32_t)entries.size(), 1u, (uint32_t)(nb * npix), 0u});
-        entries.push_back(BatchEntry{0u, 0u, ctx->spp + done, 0u});
+        entries.push_back(BatchEntry{0u, 0u, ctx->spp + done, nb});
     }
     rc = upload_tables(ctx, views, batches, entries);
     if (rc)
@@ -2047,7 +2051,7 @@ int clhip_render_views(clhip_ctx* ctx, const clhip_view* views, uint32_t nviews)
             }
             const uint32_t ns = std::min((cap - fill) / npix, ctx->vspp[i] - s0);
             BatchRec&      b  = batches.back();
-            entries.push_back(BatchEntry{i, fill, s0, 0u});
+            entries.push_back(BatchEntry{i, fill, s0, ns});
             b.nentries += 1;
             fill += ns * npix;
             b.npaths = fill;
@@ -2383,8 +2387,9 @@ int clhip_dome_tables(clhip_ctx* ctx, float* pcond, float* cdfcond, float* pv, f
 
 /* Blocks for n given rays: a thread per ray up to full residency, and as
  * many as `entries` overflow entries serve for this scene's depth (the fixed
- * scratch holds 256 blocks of the deepest tree).  With refilled lanes: 2^20 rays of the
- * 1080p scene 1.52 -> 0.39 ms, 100003 visibility queries of the spheres 160 -> 110 us). */
+ * scratch holds 256 blocks of the deepest tree).  Against the 256 blocks of
+ * one ray per lane: 2^20 rays of the 1080p scene 1.52 -> 0.39 ms, 100003
+ * visibility queries of the spheres 160 -> 110 us. */
 static uint32_t trace_rays_blocks(const clhip_ctx* ctx, uint32_t n, size_t entries)
 {
     const uint64_t want = ((uint64_t)n + 255u) / 256u, fit = entries / (256u * (size_t)stack_overflow(ctx));

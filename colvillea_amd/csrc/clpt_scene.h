@@ -201,14 +201,17 @@ struct alignas(16) ViewRec
     float    pos[4], d00[4], ddu[4], ddv[4];
 };
 
-/* A batch is a list of (view, first path, first sample) entries; path p of
- * the batch belongs to the last entry with path_begin <= p, local index
- * l = p - path_begin maps to pixel l % npix and sample sample_base + l / npix.
+/* A batch is a list of (view, first path, first sample, samples) entries;
+ * path p of the batch belongs to the last entry with path_begin <= p.  Its
+ * local index l = p - path_begin runs over groups of `group` pixels of the
+ * view (BatchTable; in tile order), within a group over the entry's samples
+ * and within a sample over the group's pixels, so that all samples of a
+ * group are traced together and find its triangles and texels in the caches.
  * The batch to run is read from *cursor, which k_batch_end advances, so a
  * captured batch graph replays unchanged. */
 struct BatchEntry
 {
-    uint32_t view, path_begin, sample_base, pad;
+    uint32_t view, path_begin, sample_base, nsamples;
 };
 
 struct BatchRec
@@ -216,12 +219,19 @@ struct BatchRec
     uint32_t entry_off, nentries, npaths, pad;
 };
 
+/* Shading waits for the texels, vertices and HDRI entries it gathers, and a
+ * group's samples gather the same ones.  1024 pixels (four 16 x 16 tiles, one
+ * window of the queues) against whole samples of the film: C1 frame at 1080p
+ * and 64 spp 77.0 -> 75.7 ms (shading 14.4 -> 13.5), 16 spp at 512 x 512
+ * 2.28 -> 2.21, 48 views 63.9 -> 62.9; 256 and 8192 pixels are within 1%. */
+#define CLPT_PIXEL_GROUP 1024u
 struct BatchTable
 {
     const ViewRec*    views;
     const BatchRec*   batches;
     const BatchEntry* entries;
     uint32_t*         cursor;
+    uint32_t          group; /* pixels whose samples are traced together */
     uint32_t          tile; /* 1: paths of a sample in pixel rows; T > 1: in T x T tiles */
 };
 

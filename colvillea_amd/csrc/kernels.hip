@@ -741,9 +741,16 @@ __device__ __forceinline__ void locate_path(const BatchTable& bt, const BatchRec
     const BatchEntry e = bt.entries[b.entry_off + lo];
     const uint32_t   n = bt.views[e.view].npix;
     const uint32_t   l = p - e.path_begin;
-    view               = e.view;
-    pixel              = l % n;
-    sample             = e.sample_base + l / n;
+    /* group g holds gn pixels (the last may be partly full), e.nsamples times;
+     * a view below one group is one group, so the product stays below npaths */
+    const uint32_t gs = min(bt.group, n);
+    const uint32_t g  = l / (gs * e.nsamples), g0 = g * gs;
+    const uint32_t r  = l - g0 * e.nsamples;
+    const uint32_t gn = min(gs, n - g0);
+    const uint32_t s  = gn == CLPT_PIXEL_GROUP ? r / CLPT_PIXEL_GROUP : r / gn;
+    view              = e.view;
+    pixel             = g0 + r - s * gn;
+    sample            = e.sample_base + s;
     if (bt.tile > 1u)
     {
         const ViewRec& v = bt.views[e.view];
@@ -1531,13 +1538,14 @@ __global__ __launch_bounds__(256) void k_film_fold(BatchTable bt, const float* p
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t en = 0; en < b.nentries; ++en)
     {
-        const BatchEntry e   = bt.entries[b.entry_off + en];
-        const ViewRec&   v   = bt.views[e.view];
-        const uint32_t   end = en + 1u < b.nentries ? bt.entries[b.entry_off + en + 1u].path_begin : b.npaths;
+        const BatchEntry e = bt.entries[b.entry_off + en];
+        const ViewRec&   v = bt.views[e.view];
         for (uint32_t l = blockIdx.x * blockDim.x + threadIdx.x; l < v.npix; l += stride)
         {
-            double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-            for (uint32_t q = e.path_begin + l; q < end; q += v.npix)
+            double         s0 = 0.0, s1 = 0.0, s2 = 0.0;
+            const uint32_t g0 = l - l % bt.group, gn = min(bt.group, v.npix - g0);
+            uint32_t       q  = e.path_begin + g0 * e.nsamples + (l - g0);
+            for (uint32_t k = 0; k < e.nsamples; ++k, q += gn)
             {
                 s0 += (double)pacc[3 * (size_t)q + 0];
                 s1 += (double)pacc[3 * (size_t)q + 1];

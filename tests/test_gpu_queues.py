@@ -2,7 +2,8 @@
 camera paths changes: films of one sample whose path counts lie around one
 window (1024 paths), one round of windows over all segments (8192) and one
 window more, against the oracle (counts exact, sums to the oracle's
-rounding), with the smallest shading grid too."""
+rounding), with the smallest shading grid too; and the order of samples
+within groups of 1024 pixels."""
 import numpy as np
 import pytest
 
@@ -35,3 +36,26 @@ def test_paths_around_a_window(size):
             # the oracle adds a path's radiances (at most 5 at depth 5) in
             # float32: at most 4 roundings of 2^-24 = 2.4e-7; the film in float64
             assert np.allclose(sums, osums, rtol=2.5e-7, atol=1e-30)
+
+
+@pytest.mark.parametrize("size", [(1, 1), (33, 31), (32, 32), (41, 25), (683, 3), (61, 41)],
+                         ids=lambda s: str(s[0] * s[1]))
+def test_samples_around_a_pixel_group(size):
+    """Several samples of films of less than one, one, just over one, just
+    over two and several groups of pixels traced together, in batches of 2,
+    2 and 1 samples and in one, in pixel rows and in tiles."""
+    w, h = size
+    desc = scenes.make_c0(width=w, height=h, spp=5, hdri_w=64, hdri_h=32)
+    with Integrator.createIntegrator(IntegratorType.WavefrontPathTracing, w, h) as integ:
+        upload_scene(integ, desc)
+        osums, ocnt = orc.Scene(desc, tables=_gpu_tables(integ, desc)).render("f32", samples=(0, 5))
+        D = desc.max_depth + 1
+        for tile, spb in ((16, 0), (16, 2), (1, 0), (1, 2)):
+            integ.setLaunch(tile=tile)
+            integ.setParams(max_depth=desc.max_depth, rr_depth=desc.rr_depth, view=desc.view, samples_per_batch=spb)
+            integ.resetIterationIndex()
+            integ.render(5)
+            sums, cnt = integ.readbackSums(), integ.counters()
+            for k in ("rays", "hits", "shadow", "visible"):
+                assert np.array_equal(cnt[k][:D], ocnt[k][:D]), (tile, spb, k)
+            assert np.allclose(sums, osums, rtol=2.5e-7, atol=1e-30), (tile, spb)
