@@ -63,16 +63,18 @@ hipError_t HostCopier::reserve(size_t bytes)
         if (e != hipSuccess)
             return e;
     }
-    if (bytes > 2 * kPiece && threads_.empty())
-        try
-        {
-            for (unsigned k = 1; k < kThreads; ++k)
-                threads_.emplace_back([this] { work(); });
-        }
-        catch (...)
-        {
-            /* as many as could be started; the caller's thread does the rest */
-        }
+    /* a thread per piece at most: starting one costs 10 to 15 us, which a
+     * context that only makes small copies would pay for nothing */
+    const size_t want = need <= 2 * kPiece ? 0u : std::min<size_t>(kThreads, need / kPiece) - 1u;
+    try
+    {
+        while (threads_.size() < want)
+            threads_.emplace_back([this] { work(); });
+    }
+    catch (...)
+    {
+        /* as many as could be started; the caller's thread does the rest */
+    }
     return hipSuccess;
 }
 
