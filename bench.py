@@ -22,7 +22,7 @@ HBM_PEAK_GBS = 8000.0
 L2_PEAK_GBS = 8 * 16 * 128 * 2.4
 QUEUE_BYTES_PER_RAY = 32 + 16  # ray o/d float4 x2 read, hit float4 (b1, b2, instance, primitive) written
 ORIGIN_BYTES = 16  # a camera ray of a one-view render reads no origin: it is the camera position
-NODE_BYTES = {4: 128, 8: 96}  # Node4: float child boxes; Node8: byte-quantised child boxes
+NODE_BYTES = {4: 80, 8: 96}  # Node4P: half-float child boxes; Node8: byte-quantised child boxes
 TRI_BYTES = 48
 
 

@@ -171,8 +171,8 @@ int clhip_create_texture_u8(clhip_ctx* ctx, const uint8_t* data, uint32_t width,
                             int srgb, int32_t* texture_id);
 
 /* Tree width of the acceleration structures built from now on: 4 (default;
- * 128-byte nodes with float boxes) or 8 (96-byte nodes with child boxes
- * quantised to bytes).  No reference counterpart (OptiX builds its own).
+ * 80-byte nodes with half-float boxes) or 8 (96-byte nodes with child boxes
+ * quantised to bytes); the stored boxes contain the exact ones.  No reference counterpart (OptiX builds its own).
  * Results do not depend on it; changing it requires building the BLAS and
  * TLAS again. */
 int clhip_set_bvh_width(clhip_ctx* ctx, uint32_t width);
