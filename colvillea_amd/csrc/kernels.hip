@@ -844,6 +844,26 @@ struct TraceShared
     float2 ring_b[CLPT_TRACE_BLOCK]; /* o.yz */
 };
 
+/* Rays of a segment that each of its waves begins with: 64, or fewer where a
+ * quarter of the waves still serves them all (waves * result >= n whenever it
+ * is below 64, so no wave has a second chunk).  A launch of few rays lasts as
+ * long as its slowest wave, and a wave's step is longer the more lanes it has:
+ * more of the step's blocks run, and a gathered load takes a cycle per four
+ * lanes.  160 x 120 frame of 1 sample 661 -> 546 us, 321 x 241 of 4 samples
+ * 902 -> 844, 1080p frame of 1 sample 4.12 -> 4.10 ms.  Down to 4 or 8 rays
+ * 558 or 585 us.  Spreading over half of the waves slows 512 x 512 of 16
+ * samples by 0.7%, over all of them the 1080p frame of 1 sample by 7%: there
+ * the waves compete for issue. */
+#define CLPT_SPREAD     4u
+#define CLPT_SPREAD_MIN 2u
+__device__ __forceinline__ uint32_t wave_rays(uint32_t n, uint32_t waves)
+{
+    uint32_t per = 64u;
+    while (per > CLPT_SPREAD_MIN && n <= waves / CLPT_SPREAD * (per / 2u))
+        per /= 2u;
+    return per;
+}
+
 /* Block bx of gx (a multiple of CLPT_SEGS) of the closest-hit rays of a
  * depth. */
 template <int W>
@@ -869,10 +889,12 @@ __device__ __forceinline__ void trace_block(TraceShared& sm, TraverseStack& st, 
      * step. */
     const uint32_t    rl     = threadIdx.x & ~63u;
     const uint32_t    stride = gx / CLPT_SEGS * CLPT_TRACE_BLOCK;
-    uint32_t          cbase  = (uint32_t)__builtin_amdgcn_readfirstlane((int)(first - lane_id())); /* this chunk */
+    const uint32_t    per    = wave_rays(n, stride / 64u);
+    const uint32_t    wbase  = (uint32_t)__builtin_amdgcn_readfirstlane((int)(first - lane_id()));
+    uint32_t          cbase  = per < 64u ? n : wbase; /* this chunk; n: no other follows */
     uint32_t          used   = 64u; /* rays of it taken (the first go to the lanes directly) */
-    uint32_t          i      = first;
-    bool              active = i < n;
+    uint32_t          i      = wbase / 64u * per + lane_id();
+    bool              active = lane_id() < per && i < n;
     Tracer<false, W>  tr;
     if (active)
     {
@@ -1435,9 +1457,11 @@ __device__ __forceinline__ void shadow_block(TraverseStack& st, uint32_t bx, uin
     sq.x += (size_t)seg * seg_cap;
     if (sq.tag)
         sq.tag += (size_t)seg * seg_cap;
-    WavePool       pool{first - lane_id(), gx / CLPT_SEGS * CLPT_TRACE_BLOCK, 64u};
-    uint32_t       i      = first;
-    bool           active = i < n;
+    const uint32_t stride = gx / CLPT_SEGS * CLPT_TRACE_BLOCK, per = wave_rays(n, stride / 64u);
+    const uint32_t wbase  = first - lane_id();
+    WavePool       pool{per < 64u ? n : wbase, stride, 64u}; /* base n: no rays follow */
+    uint32_t       i      = wbase / 64u * per + lane_id();
+    bool           active = lane_id() < per && i < n;
     Tracer<true, W> tr;
     /* the ray's radiance and pixel, read with the ray so that a visible ray's
      * film update needs no load when it finishes */

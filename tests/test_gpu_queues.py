@@ -3,7 +3,7 @@ camera paths changes: films of one sample whose path counts lie around one
 window (1024 paths), one round of windows over all segments (8192) and one
 window more, against the oracle (counts exact, sums to the oracle's
 rounding), with the smallest shading grid too; and the order of samples
-within groups of 1024 pixels."""
+within groups of 1024 pixels, and the rays that a wave begins with."""
 import numpy as np
 import pytest
 
@@ -59,3 +59,25 @@ def test_samples_around_a_pixel_group(size):
             for k in ("rays", "hits", "shadow", "visible"):
                 assert np.array_equal(cnt[k][:D], ocnt[k][:D]), (tile, spb, k)
             assert np.allclose(sums, osums, rtol=2.5e-7, atol=1e-30), (tile, spb)
+
+
+@pytest.mark.parametrize("size", [(1, 1), (8, 8), (13, 5), (51, 5), (16, 16), (257, 1), (32, 16), (27, 19), (128, 64), (8193, 1)],
+                         ids=lambda s: str(s[0] * s[1]))
+def test_rays_spread_over_waves(size):
+    """Segments whose ray counts lie around the limits below which a wave
+    begins with 2 to 32 rays: with one traversal block per CU of 256, a
+    segment has 128 waves and the limits are 64, 128, 256, 512 and 1024."""
+    w, h = size
+    desc = scenes.make_c0(width=w, height=h, spp=1, hdri_w=64, hdri_h=32)
+    with Integrator.createIntegrator(IntegratorType.WavefrontPathTracing, w, h) as integ:
+        upload_scene(integ, desc)
+        osums, ocnt = orc.Scene(desc, tables=_gpu_tables(integ, desc)).render("f32", samples=(0, 1))
+        D = desc.max_depth + 1
+        for blocks in (0, 1, 2):
+            integ.setLaunch(trace_blocks_per_cu=blocks, shadow_blocks_per_cu=blocks)
+            integ.resetIterationIndex()
+            integ.render(1)
+            sums, cnt = integ.readbackSums(), integ.counters()
+            for k in ("rays", "hits", "shadow", "visible"):
+                assert np.array_equal(cnt[k][:D], ocnt[k][:D]), (blocks, k)
+            assert np.allclose(sums, osums, rtol=2.5e-7, atol=1e-30), blocks
