@@ -26,42 +26,46 @@ HostCopier::~HostCopier()
         (void)hipHostFree(stage_);
 }
 
-hipError_t HostCopier::reserve(size_t bytes)
+bool HostCopier::reserve(size_t bytes)
 {
+    if (refused_)
+        return false;
     /* an upload may still be reading the staging */
     if (up_pending_)
     {
-        const hipError_t e = hipEventSynchronize(up_);
-        if (e != hipSuccess)
-            return e;
+        (void)hipEventSynchronize(up_);
         up_pending_ = false;
     }
     const size_t need = std::min(kStage, std::max<size_t>((bytes + kPiece - 1) / kPiece * kPiece, kPiece));
+    hipError_t   e    = hipSuccess;
     if (need > cap_)
     {
         if (stage_)
             (void)hipHostFree(stage_);
-        stage_       = nullptr;
-        cap_         = 0;
-        void*      p = nullptr;
-        hipError_t e = hipHostMalloc(&p, need, hipHostMallocDefault);
-        if (e != hipSuccess)
-            return e;
-        stage_ = static_cast<char*>(p);
-        cap_   = need;
-    }
-    for (size_t k = 0; k < need / kPiece; ++k)
-        if (!ev_[k])
+        stage_  = nullptr;
+        cap_    = 0;
+        void* p = nullptr;
+        e       = hipHostMalloc(&p, need, hipHostMallocDefault);
+        if (e == hipSuccess)
         {
-            const hipError_t e = hipEventCreateWithFlags(&ev_[k], hipEventDisableTiming);
-            if (e != hipSuccess)
-                return e;
+            stage_ = static_cast<char*>(p);
+            cap_   = need;
         }
-    if (!up_)
+    }
+    for (size_t k = 0; k < need / kPiece && e == hipSuccess; ++k)
+        if (!ev_[k])
+            e = hipEventCreateWithFlags(&ev_[k], hipEventDisableTiming);
+    if (e == hipSuccess && !up_)
+        e = hipEventCreateWithFlags(&up_, hipEventDisableTiming);
+    if (e != hipSuccess)
     {
-        const hipError_t e = hipEventCreateWithFlags(&up_, hipEventDisableTiming);
-        if (e != hipSuccess)
-            return e;
+        (void)hipGetLastError(); /* not for the next launch to report */
+        if (stage_)
+            (void)hipHostFree(stage_);
+        stage_   = nullptr;
+        cap_     = 0;
+        refused_ = true;
+        return false;
     }
     /* a thread per piece at most: starting one costs 10 to 15 us, which a
      * context that only makes small copies would pay for nothing */
@@ -75,7 +79,7 @@ hipError_t HostCopier::reserve(size_t bytes)
     {
         /* as many as could be started; the caller's thread does the rest */
     }
-    return hipSuccess;
+    return true;
 }
 
 void HostCopier::work()
@@ -134,9 +138,12 @@ hipError_t HostCopier::to_host(hipStream_t s, void* dst, const void* dev, size_t
 {
     if (!bytes)
         return hipStreamSynchronize(s);
-    hipError_t e = reserve(bytes);
-    if (e != hipSuccess)
-        return e;
+    hipError_t e;
+    if (!reserve(bytes))
+    {
+        e = hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, s);
+        return e == hipSuccess ? hipStreamSynchronize(s) : e;
+    }
     char*       out = static_cast<char*>(dst);
     const char* in  = static_cast<const char*>(dev);
     for (size_t at = 0; at < bytes; at += cap_)
@@ -174,9 +181,12 @@ hipError_t HostCopier::from_host(hipStream_t s, void* dev, const void* src, size
     char*       out = static_cast<char*>(dev);
     for (size_t at = 0; at < bytes; at += cap_)
     {
-        hipError_t e = reserve(bytes);
-        if (e != hipSuccess)
-            return e;
+        hipError_t e;
+        if (!reserve(bytes)) /* never after a part was staged */
+        {
+            e = hipMemcpyAsync(dev, src, bytes, hipMemcpyHostToDevice, s);
+            return e == hipSuccess ? hipStreamSynchronize(s) : e; /* src may be reused */
+        }
         const size_t part = std::min(cap_, bytes - at);
         run((part + kPiece - 1) / kPiece, [&](size_t k) {
             std::memcpy(stage_ + k * kPiece, in + at + k * kPiece, std::min(kPiece, part - k * kPiece));

@@ -22,7 +22,8 @@ namespace clpt
  * kThreads threads copy them out as they arrive.  One HostCopier serves one
  * context (it is not thread-safe); it holds at most kStage bytes of pinned
  * memory and its threads, both made at the first copy that needs them and
- * kept for the context's life. */
+ * kept for the context's life.  Where no pinned memory can be had, copies go
+ * the runtime's way. */
 class HostCopier
 {
 public:
@@ -43,7 +44,8 @@ private:
     static constexpr size_t   kStage   = kPiece * kSlots;
     static constexpr unsigned kThreads = 8; /* the caller's among them */
 
-    hipError_t reserve(size_t bytes);
+    /* staging, events and threads for a copy; false: there are none to be had */
+    bool reserve(size_t bytes);
     /* job(k) for k = 0..n-1 on the threads; returns when all are done */
     void run(size_t n, const std::function<void(size_t)>& job);
     void work();
@@ -51,6 +53,7 @@ private:
     int                      device_;
     char*                    stage_ = nullptr;
     size_t                   cap_   = 0;
+    bool                     refused_ = false; /* pinned memory or an event could not be had */
     hipEvent_t               ev_[kSlots] = {};
     hipEvent_t               up_ = nullptr; /* the last from_host transfer */
     bool                     up_pending_ = false;
