@@ -15,8 +15,7 @@ HostCopier::~HostCopier()
     wake_.notify_all();
     for (std::thread& t : threads_)
         t.join();
-    if (up_pending_)
-        (void)hipEventSynchronize(up_);
+    wait_upload();
     for (hipEvent_t e : ev_)
         if (e)
             (void)hipEventDestroy(e);
@@ -26,16 +25,32 @@ HostCopier::~HostCopier()
         (void)hipHostFree(stage_);
 }
 
+/* Whether p is ordinary memory, which the runtime would copy through staging
+ * of its own; pinned and managed memory it reads and writes directly. */
+static bool pageable(const void* p)
+{
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeUnregistered;
+}
+
+/* An upload may still be reading the staging. */
+void HostCopier::wait_upload()
+{
+    if (up_pending_)
+        (void)hipEventSynchronize(up_);
+    up_pending_ = false;
+}
+
 bool HostCopier::reserve(size_t bytes)
 {
     if (refused_)
         return false;
-    /* an upload may still be reading the staging */
-    if (up_pending_)
-    {
-        (void)hipEventSynchronize(up_);
-        up_pending_ = false;
-    }
+    wait_upload();
     const size_t need = std::min(kStage, std::max<size_t>((bytes + kPiece - 1) / kPiece * kPiece, kPiece));
     hipError_t   e    = hipSuccess;
     if (need > cap_)
@@ -139,7 +154,7 @@ hipError_t HostCopier::to_host(hipStream_t s, void* dst, const void* dev, size_t
     if (!bytes)
         return hipStreamSynchronize(s);
     hipError_t e;
-    if (!reserve(bytes))
+    if (!pageable(dst) || !reserve(bytes))
     {
         e = hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
@@ -177,16 +192,19 @@ hipError_t HostCopier::to_host(hipStream_t s, void* dst, const void* dev, size_t
 
 hipError_t HostCopier::from_host(hipStream_t s, void* dev, const void* src, size_t bytes)
 {
+    if (!bytes)
+        return hipSuccess;
+    hipError_t e;
+    if (!pageable(src) || !reserve(bytes))
+    {
+        e = hipMemcpyAsync(dev, src, bytes, hipMemcpyHostToDevice, s);
+        return e == hipSuccess ? hipStreamSynchronize(s) : e; /* src may be reused */
+    }
     const char* in  = static_cast<const char*>(src);
     char*       out = static_cast<char*>(dev);
     for (size_t at = 0; at < bytes; at += cap_)
     {
-        hipError_t e;
-        if (!reserve(bytes)) /* never after a part was staged */
-        {
-            e = hipMemcpyAsync(dev, src, bytes, hipMemcpyHostToDevice, s);
-            return e == hipSuccess ? hipStreamSynchronize(s) : e; /* src may be reused */
-        }
+        wait_upload();
         const size_t part = std::min(cap_, bytes - at);
         run((part + kPiece - 1) / kPiece, [&](size_t k) {
             std::memcpy(stage_ + k * kPiece, in + at + k * kPiece, std::min(kPiece, part - k * kPiece));

@@ -22,8 +22,9 @@ namespace clpt
  * kThreads threads copy them out as they arrive.  One HostCopier serves one
  * context (it is not thread-safe); it holds at most kStage bytes of pinned
  * memory and its threads, both made at the first copy that needs them and
- * kept for the context's life.  Where no pinned memory can be had, copies go
- * the runtime's way. */
+ * kept for the context's life.  Copies to and
+ * from memory that is not pageable, and all copies where no pinned memory can
+ * be had, go the runtime's way. */
 class HostCopier
 {
 public:
@@ -46,6 +47,7 @@ private:
 
     /* staging, events and threads for a copy; false: there are none to be had */
     bool reserve(size_t bytes);
+    void wait_upload();
     /* job(k) for k = 0..n-1 on the threads; returns when all are done */
     void run(size_t n, const std::function<void(size_t)>& job);
     void work();

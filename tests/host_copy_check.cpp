@@ -226,6 +226,24 @@ int main(int argc, char** argv)
             expect(staged_copies == 0, "staged copies", staged_copies, 0);
             refuse_pinned = false;
         }
+        else if (what == "pinned")
+        {
+            /* the caller's own pinned memory is written and read directly */
+            const size_t n = 5 * MiB + 3;
+            void*        own = nullptr;
+            (void)hipHostMalloc(&own, n, 0);
+            const std::vector<char> src = bytes_of(n, 9u);
+            std::vector<char>       up(n);
+            expect(c.to_host(nullptr, own, src.data(), n) == hipSuccess, "to_host fails", n, 0);
+            expect(std::memcmp(own, src.data(), n) == 0, "to_host differs", n, 0);
+            expect(c.from_host(nullptr, up.data(), own, n) == hipSuccess, "from_host fails", n, 0);
+            std::memset(own, 0, n); /* src may be reused on return */
+            (void)hipStreamSynchronize(nullptr);
+            expect(std::memcmp(up.data(), src.data(), n) == 0, "from_host differs", n, 0);
+            expect(staged_copies == 2 && direct_copies == 0, "copies", staged_copies, direct_copies);
+            expect(pinned_calls == 1, "pinned allocations", pinned_calls, 1);
+            (void)hipHostFree(own);
+        }
         else
             expect(false, "unknown case", 0, 0);
     }

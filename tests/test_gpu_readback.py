@@ -4,10 +4,14 @@ linear film equals the float64 sums over the samples, and both equal the film
 of a batched render of the same view.  Twice in a row with other samples, so
 that a stale piece shows.  Training samples take the same way up: one Adam
 step on a large batch equals the step on the same samples in a fresh context."""
+import ctypes as C
+
 import numpy as np
 import pytest
+import torch
 
 from colvillea_amd import Integrator, IntegratorType, scenes, upload_scene
+from colvillea_amd import _capi as capi
 from colvillea_amd.integrator import View
 
 pytestmark = pytest.mark.gpu
@@ -32,6 +36,18 @@ def test_film_readback(size):
             assert np.array_equal(img[..., :3], (sums * 0.5).astype(np.float32))
             assert np.all(img[..., 3] == 1.0)
             assert np.allclose(integ.readbackView(0), img, rtol=1e-6, atol=0)
+
+
+def test_readback_into_pinned_memory():
+    w, h = 512, 300  # 2.3 MiB
+    desc = scenes.make_c0(width=w, height=h, spp=1, hdri_w=64, hdri_h=32)
+    out = torch.zeros((h, w, 4), dtype=torch.float32, pin_memory=True)
+    with Integrator.createIntegrator(IntegratorType.WavefrontPathTracing, w, h) as integ:
+        upload_scene(integ, desc)
+        integ.render(1)
+        capi.check(capi.lib().clhip_readback(integ.ctx, C.cast(out.data_ptr(), C.POINTER(C.c_float)), out.numel() * 4),
+                   integ.ctx)
+        assert np.array_equal(out.numpy(), integ.readbackFramebufferLinear())
 
 
 @pytest.mark.parametrize("n", [1, 20165, 20166, 60000, 700001])

@@ -23,7 +23,8 @@ def exe(tmp_path_factory):
 
 # sizes: every size arrives whole, up and down
 # no_pinned: without pinned memory copies still work
-@pytest.mark.parametrize("case", ["sizes", "no_pinned"])
+# pinned: the caller's own pinned memory takes one copy, not two
+@pytest.mark.parametrize("case", ["sizes", "no_pinned", "pinned"])
 def test_copies(exe, case):
     r = subprocess.run([exe, case], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
