@@ -176,6 +176,12 @@ hipError_t HostCopier::to_host(hipStream_t s, void* dst, const void* dev, size_t
                 return e;
             }
         }
+        /* the copies lie behind all of the stream's work, a whole render
+         * perhaps: the caller's thread waits for that alone, and the others
+         * wake to transfers in progress (an event wait polls) */
+        e = hipEventSynchronize(ev_[0]);
+        if (e != hipSuccess)
+            return e;
         std::atomic<int> bad{(int)hipSuccess};
         run(n, [&](size_t k) {
             const hipError_t w = hipEventSynchronize(ev_[k]);

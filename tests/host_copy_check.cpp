@@ -244,6 +244,28 @@ int main(int argc, char** argv)
             expect(pinned_calls == 1, "pinned allocations", pinned_calls, 1);
             (void)hipHostFree(own);
         }
+        else if (what == "wait")
+        {
+            /* a readback behind a render in progress: one thread waits */
+            set_gate(false);
+            const size_t            n = 24 * MiB + 5;
+            const std::vector<char> src = bytes_of(n, 5u);
+            std::vector<char>       out(n);
+            std::thread             caller([&] {
+                expect(c.to_host(nullptr, out.data(), src.data(), n) == hipSuccess, "to_host fails", n, 0);
+            });
+            int most = 0;
+            for (int k = 0; k < 100; ++k)
+            {
+                std::this_thread::sleep_for(std::chrono::milliseconds(2));
+                std::lock_guard<std::mutex> l(mu);
+                most = std::max(most, waiting);
+            }
+            expect(most == 1, "threads waiting for the render", (size_t)most, 1);
+            set_gate(true);
+            caller.join();
+            expect(out == src, "to_host differs", n, 0);
+        }
         else
             expect(false, "unknown case", 0, 0);
     }
