@@ -15,12 +15,12 @@ HostCopier::~HostCopier()
     wake_.notify_all();
     for (std::thread& t : threads_)
         t.join();
-    wait_upload();
-    for (hipEvent_t e : ev_)
-        if (e)
-            (void)hipEventDestroy(e);
-    if (up_)
-        (void)hipEventDestroy(up_);
+    for (size_t k = 0; k < kSlots; ++k)
+    {
+        wait_upload(k);
+        if (ev_[k])
+            (void)hipEventDestroy(ev_[k]);
+    }
     if (stage_)
         (void)hipHostFree(stage_);
 }
@@ -38,68 +38,67 @@ static bool pageable(const void* p)
     return a.type == hipMemoryTypeUnregistered;
 }
 
-/* An upload may still be reading the staging. */
-void HostCopier::wait_upload()
+/* An upload may still be reading slot k. */
+void HostCopier::wait_upload(size_t k)
 {
-    if (up_pending_)
-        (void)hipEventSynchronize(up_);
-    up_pending_ = false;
+    if (up_pending_[k])
+        (void)hipEventSynchronize(ev_[k]);
+    up_pending_[k] = false;
 }
 
 bool HostCopier::reserve(size_t bytes)
 {
     if (refused_)
         return false;
-    wait_upload();
-    const size_t need = std::min(kStage, std::max<size_t>((bytes + kPiece - 1) / kPiece * kPiece, kPiece));
+    for (size_t k = 0; k < kSlots; ++k)
+        wait_upload(k);
+    const size_t need = std::min(kSlots, (bytes + kPart - 1) / kPart);
     hipError_t   e    = hipSuccess;
-    if (need > cap_)
+    bool         fresh = false;
+    if (need > slots_)
     {
         if (stage_)
             (void)hipHostFree(stage_);
         stage_  = nullptr;
-        cap_    = 0;
+        slots_  = 0;
         void* p = nullptr;
-        e       = hipHostMalloc(&p, need, hipHostMallocDefault);
+        e       = hipHostMalloc(&p, need * kPart, hipHostMallocDefault);
         if (e == hipSuccess)
         {
             stage_ = static_cast<char*>(p);
-            cap_   = need;
+            slots_ = need;
+            fresh  = true;
         }
     }
-    for (size_t k = 0; k < need / kPiece && e == hipSuccess; ++k)
+    for (size_t k = 0; k < need && e == hipSuccess; ++k)
         if (!ev_[k])
             e = hipEventCreateWithFlags(&ev_[k], hipEventDisableTiming);
-    if (e == hipSuccess && !up_)
-        e = hipEventCreateWithFlags(&up_, hipEventDisableTiming);
     if (e != hipSuccess)
     {
         (void)hipGetLastError(); /* not for the next launch to report */
         if (stage_)
             (void)hipHostFree(stage_);
         stage_   = nullptr;
-        cap_     = 0;
+        slots_   = 0;
         refused_ = true;
         return false;
     }
-    /* a thread per piece at most: starting one costs 10 to 15 us, which a
-     * context that only makes small copies would pay for nothing */
-    const size_t want = need <= 2 * kPiece ? 0u : std::min<size_t>(kThreads, need / kPiece) - 1u;
-    try
+    if (fresh)
     {
-        while (threads_.size() < want)
-            threads_.emplace_back([this] { work(); });
-    }
-    catch (...)
-    {
-        /* as many as could be started; the caller's thread does the rest */
+        /* its pages are mapped as the host first touches them, 100 us and
+         * more per MiB; the stream's work goes on meanwhile */
+        const std::function<void(size_t)> touch = [&](size_t i) {
+            for (size_t at = 0; at < kPiece; at += 4096)
+                *static_cast<volatile char*>(stage_ + i * kPiece + at) = 0;
+        };
+        begin(slots_ * kPer, touch);
+        finish();
     }
     return true;
 }
 
 void HostCopier::work()
 {
-    (void)hipSetDevice(device_);
     uint64_t seen = 0;
     for (;;)
     {
@@ -125,13 +124,18 @@ void HostCopier::work()
     }
 }
 
-void HostCopier::run(size_t n, const std::function<void(size_t)>& job)
+void HostCopier::begin(size_t n, const std::function<void(size_t)>& job)
 {
-    if (n < 3 || threads_.empty())
+    /* a thread per MiB at most: starting one costs 10 to 15 us */
+    const size_t want = std::min<size_t>(kThreads, n * kPiece >> 20);
+    try
     {
-        for (size_t k = 0; k < n; ++k)
-            job(k);
-        return;
+        while (threads_.size() + 1 < want)
+            threads_.emplace_back([this] { work(); });
+    }
+    catch (...)
+    {
+        /* as many as could be started; the caller's thread does the rest */
     }
     {
         std::lock_guard<std::mutex> l(mu_);
@@ -141,8 +145,18 @@ void HostCopier::run(size_t n, const std::function<void(size_t)>& job)
         ++round_;
     }
     wake_.notify_all();
-    for (size_t k = next_++; k < n; k = next_++)
-        job(k);
+}
+
+void HostCopier::help(size_t end)
+{
+    for (size_t k = next_; k < end; k = next_)
+        if (next_.compare_exchange_weak(k, k + 1))
+            (*job_)(k);
+}
+
+void HostCopier::finish()
+{
+    help(njobs_);
     /* no thread takes the job up any more, and those that did are done */
     std::unique_lock<std::mutex> l(mu_);
     job_ = nullptr;
@@ -153,78 +167,114 @@ hipError_t HostCopier::to_host(hipStream_t s, void* dst, const void* dev, size_t
 {
     if (!bytes)
         return hipStreamSynchronize(s);
-    hipError_t e;
-    if (!pageable(dst) || !reserve(bytes))
+    hipError_t e = hipSuccess;
+    if (bytes < kMin || !pageable(dst) || !reserve(bytes))
     {
         e = hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
-    char*       out = static_cast<char*>(dst);
-    const char* in  = static_cast<const char*>(dev);
-    for (size_t at = 0; at < bytes; at += cap_)
+    char*        out    = static_cast<char*>(dst);
+    const char*  in     = static_cast<const char*>(dev);
+    const size_t parts  = (bytes + kPart - 1) / kPart, pieces = (bytes + kPiece - 1) / kPiece;
+    const auto   end_of = [&](size_t p) { return std::min(pieces, (p + 1) * kPer); };
+    const auto   queue  = [&](size_t p) {
+        const size_t k = p % slots_;
+        left_[k]       = end_of(p) - p * kPer;
+        const hipError_t q =
+            hipMemcpyAsync(stage_ + k * kPart, in + p * kPart, std::min(kPart, bytes - p * kPart), hipMemcpyDeviceToHost, s);
+        return q == hipSuccess ? hipEventRecord(ev_[k], s) : q;
+    };
+    std::atomic<size_t> arrived{0}; /* parts */
+    std::atomic<bool>   failed{false};
+    const std::function<void(size_t)> job = [&](size_t i) {
+        const size_t p = i / kPer;
+        while (arrived.load(std::memory_order_acquire) <= p)
+            std::this_thread::yield();
+        if (!failed)
+            std::memcpy(out + i * kPiece, stage_ + p % slots_ * kPart + i % kPer * kPiece, std::min(kPiece, bytes - i * kPiece));
+        left_[p % slots_].fetch_sub(1, std::memory_order_release);
+    };
+    for (size_t p = 0; p < std::min(slots_, parts) && e == hipSuccess; ++p)
+        e = queue(p);
+    /* The copies lie behind all of the stream's work, a whole render perhaps:
+     * the caller's thread waits for that alone, and the others wake to
+     * transfers in progress. */
+    if (e == hipSuccess)
+        e = hipEventSynchronize(ev_[0]);
+    if (e == hipSuccess)
     {
-        const size_t part = std::min(cap_, bytes - at), n = (part + kPiece - 1) / kPiece;
-        for (size_t k = 0; k < n; ++k)
+        begin(pieces, job);
+        for (size_t p = 0; p < parts; ++p)
         {
-            const size_t len = std::min(kPiece, part - k * kPiece);
-            e = hipMemcpyAsync(stage_ + k * kPiece, in + at + k * kPiece, len, hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess)
-                e = hipEventRecord(ev_[k], s);
+            if (p && e == hipSuccess)
+                e = hipEventSynchronize(ev_[p % slots_]);
             if (e != hipSuccess)
+                failed = true;
+            arrived.store(p + 1, std::memory_order_release);
+            help(end_of(p));
+            if (p + slots_ < parts)
             {
-                (void)hipStreamSynchronize(s); /* the pieces queued so far */
-                return e;
+                while (left_[p % slots_].load(std::memory_order_acquire))
+                    std::this_thread::yield();
+                if (e == hipSuccess)
+                    e = queue(p + slots_);
+                else
+                    left_[p % slots_] = end_of(p + slots_) - (p + slots_) * kPer;
             }
         }
-        /* the copies lie behind all of the stream's work, a whole render
-         * perhaps: the caller's thread waits for that alone, and the others
-         * wake to transfers in progress (an event wait polls) */
-        e = hipEventSynchronize(ev_[0]);
-        if (e != hipSuccess)
-            return e;
-        std::atomic<int> bad{(int)hipSuccess};
-        run(n, [&](size_t k) {
-            const hipError_t w = hipEventSynchronize(ev_[k]);
-            if (w != hipSuccess)
-                bad = (int)w;
-            else
-                std::memcpy(out + at + k * kPiece, stage_ + k * kPiece, std::min(kPiece, part - k * kPiece));
-        });
-        if (bad != (int)hipSuccess)
-            return (hipError_t)bad.load();
+        finish();
     }
-    return hipSuccess;
+    if (e != hipSuccess)
+        (void)hipStreamSynchronize(s); /* parts still queued write the staging */
+    return e;
 }
 
 hipError_t HostCopier::from_host(hipStream_t s, void* dev, const void* src, size_t bytes)
 {
     if (!bytes)
         return hipSuccess;
-    hipError_t e;
-    if (!pageable(src) || !reserve(bytes))
+    hipError_t e = hipSuccess;
+    if (bytes < kMin || !pageable(src) || !reserve(bytes))
     {
         e = hipMemcpyAsync(dev, src, bytes, hipMemcpyHostToDevice, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e; /* src may be reused */
     }
-    const char* in  = static_cast<const char*>(src);
-    char*       out = static_cast<char*>(dev);
-    for (size_t at = 0; at < bytes; at += cap_)
+    const char*  in     = static_cast<const char*>(src);
+    char*        out    = static_cast<char*>(dev);
+    const size_t parts  = (bytes + kPart - 1) / kPart, pieces = (bytes + kPiece - 1) / kPiece;
+    const auto   end_of = [&](size_t p) { return std::min(pieces, (p + 1) * kPer); };
+    std::atomic<size_t> open{std::min(slots_, parts)}; /* parts whose slot may be written */
+    const std::function<void(size_t)> job = [&](size_t i) {
+        const size_t p = i / kPer;
+        while (open.load(std::memory_order_acquire) <= p)
+            std::this_thread::yield();
+        std::memcpy(stage_ + p % slots_ * kPart + i % kPer * kPiece, in + i * kPiece, std::min(kPiece, bytes - i * kPiece));
+        left_[p % slots_].fetch_sub(1, std::memory_order_release);
+    };
+    for (size_t p = 0; p < open; ++p)
+        left_[p] = end_of(p) - p * kPer;
+    begin(pieces, job);
+    for (size_t p = 0; p < parts; ++p)
     {
-        wait_upload();
-        const size_t part = std::min(cap_, bytes - at);
-        run((part + kPiece - 1) / kPiece, [&](size_t k) {
-            std::memcpy(stage_ + k * kPiece, in + at + k * kPiece, std::min(kPiece, part - k * kPiece));
-        });
-        e = hipMemcpyAsync(out + at, stage_, part, hipMemcpyHostToDevice, s);
+        const size_t k = p % slots_;
+        help(end_of(p));
+        while (left_[k].load(std::memory_order_acquire))
+            std::this_thread::yield();
         if (e == hipSuccess)
-            e = hipEventRecord(up_, s);
-        if (e != hipSuccess)
+            e = hipMemcpyAsync(out + p * kPart, stage_ + k * kPart, std::min(kPart, bytes - p * kPart), hipMemcpyHostToDevice, s);
+        if (e == hipSuccess)
+            e = hipEventRecord(ev_[k], s);
+        up_pending_[k] = e == hipSuccess;
+        if (p + slots_ < parts)
         {
-            (void)hipStreamSynchronize(s);
-            return e;
+            wait_upload(k);
+            left_[k] = end_of(p + slots_) - (p + slots_) * kPer;
+            open.store(p + slots_ + 1, std::memory_order_release);
         }
-        up_pending_ = true;
     }
-    return hipSuccess;
+    finish();
+    if (e != hipSuccess)
+        (void)hipStreamSynchronize(s);
+    return e;
 }
 } // namespace clpt

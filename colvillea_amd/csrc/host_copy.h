@@ -15,20 +15,27 @@
 
 namespace clpt
 {
-/* The runtime's own copy to pageable memory goes through its staging 1 MB at
- * a time, 20 us of transfer and then 70 us in one thread that copies the
- * piece and faults its pages in: 2.9 ms for a 1080p RGBA32F film.  Here the
- * pieces of a copy are queued on the stream together, into pinned slots, and
- * kThreads threads copy them out as they arrive.  One HostCopier serves one
- * context (it is not thread-safe); it holds at most kStage bytes of pinned
- * memory and its threads, both made at the first copy that needs them and
- * kept for the context's life.  Copies to and
- * from memory that is not pageable, and all copies where no pinned memory can
- * be had, go the runtime's way. */
+/* The runtime's own copy to pageable memory moves 1 MB at a time through one
+ * thread.  Here a copy is queued on the stream in parts of 2 MiB into two
+ * pinned slots, and kThreads threads copy the parts out (or in) as they
+ * arrive; a slot is queued again as soon as it is empty.  Copies below kMin,
+ * copies to and from memory that is not pageable, and all copies where no
+ * pinned memory can be had, go the runtime's way.
+ *
+ * One HostCopier serves one context (it is not thread-safe).  Its staging and
+ * threads are made at the first copy that needs them and kept for the
+ * context's life; new pinned memory costs a multiple of what a copy through
+ * it does until the host has touched it (100 us and more per MiB with all
+ * threads), so there is little of it.  Film of 1920x1080 (31.6 MiB) read back
+ * after a render, first and later times in a context: 1.9 and 1.9 ms through
+ * the runtime, 3.1 and 1.08 with 32 slots of 1 MiB each queued once, 0.89 and
+ * 0.85 with these two; two slots of 1 MiB 1.07 later, of 4 MiB or four of 2
+ * MiB no faster and up to 1 ms longer the first time.  Below kMin the threads
+ * gain nothing: 1.2 MiB takes 97 us either way, 0.3 MiB 39 against 45. */
 class HostCopier
 {
 public:
-    explicit HostCopier(int device) : device_(device) {}
+    HostCopier() = default;
     ~HostCopier();
     HostCopier(const HostCopier&) = delete;
     HostCopier& operator=(const HostCopier&) = delete;
@@ -40,25 +47,30 @@ public:
     hipError_t from_host(hipStream_t s, void* dev, const void* src, size_t bytes);
 
 private:
-    static constexpr size_t   kPiece   = 1u << 20;
-    static constexpr size_t   kSlots   = 32;
-    static constexpr size_t   kStage   = kPiece * kSlots;
+    static constexpr size_t   kMin     = 2u << 20;
+    static constexpr size_t   kPart    = 2u << 20; /* one transfer, one slot */
+    static constexpr size_t   kSlots   = 2;
+    static constexpr size_t   kPiece   = 128u << 10; /* what a thread copies at a time */
+    static constexpr size_t   kPer     = kPart / kPiece;
     static constexpr unsigned kThreads = 8; /* the caller's among them */
 
-    /* staging, events and threads for a copy; false: there are none to be had */
+    /* staging and events for a copy; false: there are none to be had */
     bool reserve(size_t bytes);
-    void wait_upload();
-    /* job(k) for k = 0..n-1 on the threads; returns when all are done */
-    void run(size_t n, const std::function<void(size_t)>& job);
+    void wait_upload(size_t k);
+    /* job(k) for k = 0..n-1 on the threads from begin() on; the caller's takes
+     * those below `end` that are left in help() and all in finish(), which
+     * returns when all are done */
+    void begin(size_t n, const std::function<void(size_t)>& job);
+    void help(size_t end);
+    void finish();
     void work();
 
-    int                      device_;
     char*                    stage_ = nullptr;
-    size_t                   cap_   = 0;
+    size_t                   slots_ = 0;
     bool                     refused_ = false; /* pinned memory or an event could not be had */
-    hipEvent_t               ev_[kSlots] = {};
-    hipEvent_t               up_ = nullptr; /* the last from_host transfer */
-    bool                     up_pending_ = false;
+    hipEvent_t               ev_[kSlots] = {}; /* the last transfer of each slot */
+    bool                     up_pending_[kSlots] = {}; /* it was an upload and may not be done */
+    std::atomic<size_t>      left_[kSlots] = {}; /* pieces of the slot's part still to be copied */
     std::vector<std::thread> threads_;
     std::mutex               mu_;
     std::condition_variable  wake_, idle_;

@@ -163,7 +163,6 @@ hipError_t hipStreamSynchronize(hipStream_t)
     wait_for(at);
     return hipSuccess;
 }
-hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipGetLastError(void)
 {
     std::lock_guard<std::mutex> l(mu);
@@ -205,14 +204,14 @@ int main(int argc, char** argv)
     const std::string what = argc > 1 ? argv[1] : "";
     std::thread       dev(device);
     {
-        HostCopier c(0);
+        HostCopier c;
         if (what == "sizes")
         {
             /* around pieces, the sizes from which several threads copy, the
              * whole staging and several times it, up and down in turn */
-            for (size_t n : {(size_t)0, (size_t)1, MiB - 1, MiB, MiB + 1, 2 * MiB - 1, 2 * MiB, 2 * MiB + 1, 3 * MiB + 7,
-                             4 * MiB, 4 * MiB + 1, 8 * MiB - 1, 8 * MiB, 8 * MiB + 1, 12 * MiB + 5, 16 * MiB, 32 * MiB + 3,
-                             70 * MiB + 1, 5 * MiB, (size_t)100})
+            for (size_t n : {(size_t)0, (size_t)1, MiB, 2 * MiB - 1, 2 * MiB, 2 * MiB + 1, 5 * MiB / 2, 3 * MiB + 7, 4 * MiB,
+                             4 * MiB + 1, 8 * MiB - 1, 8 * MiB, 8 * MiB + 1, 17 * MiB / 2, 12 * MiB, 12 * MiB + 5, 16 * MiB,
+                             32 * MiB + 3, 70 * MiB + 1, 5 * MiB, (size_t)100})
                 both_ways(c, n, (uint32_t)n + 1u);
         }
         else if (what == "no_pinned")
@@ -265,6 +264,15 @@ int main(int argc, char** argv)
             set_gate(true);
             caller.join();
             expect(out == src, "to_host differs", n, 0);
+        }
+        else if (what == "setup")
+        {
+            /* small copies make no staging; no copy makes more than 4 MiB */
+            for (size_t n : {(size_t)1, MiB, 2 * MiB - 1})
+                both_ways(c, n, 4u);
+            expect(pinned_calls == 0, "pinned allocations of small copies", pinned_calls, 0);
+            both_ways(c, 70 * MiB + 1, 4u);
+            expect(pinned_total <= 4 * MiB, "staging", pinned_total, 4 * MiB);
         }
         else
             expect(false, "unknown case", 0, 0);

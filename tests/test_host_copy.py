@@ -25,7 +25,8 @@ def exe(tmp_path_factory):
 # no_pinned: without pinned memory copies still work
 # pinned: the caller's own pinned memory takes one copy, not two
 # wait: behind a render still running only the calling thread waits
-@pytest.mark.parametrize("case", ["sizes", "no_pinned", "pinned", "wait"])
+# setup: small copies make no staging, large ones a bounded one
+@pytest.mark.parametrize("case", ["sizes", "no_pinned", "pinned", "wait", "setup"])
 def test_copies(exe, case):
     r = subprocess.run([exe, case], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
