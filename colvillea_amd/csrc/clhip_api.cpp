@@ -190,7 +190,7 @@ struct clhip_ctx
     clhip_guide guide{};
     bool        guide_ready = false;
     DevBuf      g_params, g_m1, g_m2, g_W, g_WT, g_img, g_gc, g_img8, g_scl;
-    DevBuf      g_raw, g_gradout; /* clhip_guide_train: the caller's samples, the gradient */
+    DevBuf      g_gradout; /* clhip_guide_train: the gradient, where one was asked for */
     DevBuf      g_X, g_act[4], g_out, g_grad[5], g_loss, g_wpart, g_spart, g_amaxp, g_partial, g_samples;
     uint32_t    g_partcap = 0; /* blocks the per-block gradient buffers hold */
     uint32_t    g_N = 0;
@@ -2775,13 +2775,15 @@ int clhip_guide_train(clhip_ctx* ctx, const float* s13, uint32_t n, float* grad,
     int            rc = guide_train_buffers(ctx, N);
     if (rc)
         return rc;
-    if ((size_t)n * 13 * sizeof(float) > ctx->g_raw.bytes)
-        CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream)); /* about to move */
-    CLHIP_CHECK(ctx, ctx->g_raw.alloc((size_t)n * 13 * sizeof(float)));
-    CLHIP_CHECK(ctx, ctx->g_gradout.alloc(CLPT_G_PARAMS * sizeof(float)));
-    CLHIP_CHECK(ctx, ctx->copier->from_host(ctx->stream, ctx->g_raw.p, s13, (size_t)n * 13 * sizeof(float)));
-    CLHIP_CHECK(ctx, clpt::launch_guide_samples(ctx->stream, ctx->g_raw.as<const float>(), n, ctx->g_samples.as<GuideSample>(),
+    /* the caller's rows land in the features' buffer (512 bytes a sample),
+     * which a step writes after they are unpacked, if at all */
+    float* const raw = ctx->g_X.as<float>();
+    static_assert(13 * sizeof(float) <= CLPT_G_IN * sizeof(__bf16), "a sample's row fits its features");
+    CLHIP_CHECK(ctx, ctx->copier->from_host(ctx->stream, raw, s13, (size_t)n * 13 * sizeof(float)));
+    CLHIP_CHECK(ctx, clpt::launch_guide_samples(ctx->stream, raw, n, ctx->g_samples.as<GuideSample>(),
                                                 ctx->g_gc.as<GuideCounters>()));
+    if (grad)
+        CLHIP_CHECK(ctx, ctx->g_gradout.alloc(CLPT_G_PARAMS * sizeof(float)));
     if (grad) /* a step without samples leaves it unwritten */
         CLHIP_CHECK(ctx, hipMemsetAsync(ctx->g_gradout.p, 0, CLPT_G_PARAMS * sizeof(float), ctx->stream));
     CLHIP_CHECK(ctx, clpt::launch_guide_train(ctx->stream, guide_bufs(ctx), N,

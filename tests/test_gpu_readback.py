@@ -3,13 +3,15 @@ the two pieces from which several threads copy, and its 32 MiB of slots: the
 linear film equals the float64 sums over the samples, and both equal the film
 of a batched render of the same view.  Twice in a row with other samples, so
 that a stale piece shows.  Training samples take the same way up: one Adam
-step on a large batch equals the step on the same samples in a fresh context."""
+step on a large batch equals the step on the same samples in a fresh context,
+and the loss of the rows at the edges of the copy's parts is the oracle's."""
 import ctypes as C
 
 import numpy as np
 import pytest
 import torch
 
+import guide_ref as G
 from colvillea_amd import Integrator, IntegratorType, scenes, upload_scene
 from colvillea_amd import _capi as capi
 from colvillea_amd.integrator import View
@@ -50,7 +52,7 @@ def test_readback_into_pinned_memory():
         assert np.array_equal(out.numpy(), integ.readbackFramebufferLinear())
 
 
-@pytest.mark.parametrize("n", [1, 20165, 20166, 60000, 700001])
+@pytest.mark.parametrize("n", [1, 20165, 20166, 40329, 40330, 60000, 80661, 700001])
 def test_training_samples_upload(n):
     rng = np.random.default_rng(n)
     unit = lambda v: v / np.linalg.norm(v, axis=1, keepdims=True)
@@ -69,3 +71,28 @@ def test_training_samples_upload(n):
     assert out[0][0] == out[1][0]
     assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][2], out[1][2])
     assert np.any(out[0][1])
+
+    # only the rows at the ends and at the first edges of 2 MiB parts carry
+    # weight: a stale piece would bring in thousands of weighted rows
+    cut = np.arange(0, 52 * n, 2 << 20)[:4] // 52
+    rows = np.unique(np.clip(np.concatenate([cut - 1, cut, cut + 1, [n - 1]]), 0, n - 1))
+    w = s[rows, 12].astype(np.float64)
+    t = s.copy()
+    t[:, 12] = 0.0
+    t[rows, 12] = s[rows, 12]
+    with Integrator.createIntegrator(IntegratorType.WavefrontPathTracing, 8, 8) as integ:
+        integ.guideReset(3)
+        integ.guideTrain(s[::-1].copy())
+        integ.guideReset(3)
+        Ws = G.split_params(integ.guideWeights().astype(np.float64))
+        Ws[4][:, :40] *= 10.0  # densities that differ from sample to sample
+        p = G.join_params(Ws).astype(np.float32)
+        integ.setGuideWeights(p)
+        loss, _ = integ.guideTrain(t)
+    out, _ = G.forward(G.split_params(p.astype(np.float64)), G.encode(t[rows, :9].astype(np.float64)), bf=True)
+    each = -np.log(G.mix_pdf(out, t[rows, 9:12].astype(np.float64)))
+    ref = (w * each).sum() / w.sum()
+    # 1e-3: the bound of the gradient test for the same bfloat16 network; one
+    # wrong row among these shifts the loss by its share of |each - ref|
+    assert abs(loss - ref) <= 1e-3 * abs(ref), (loss, ref)
+    assert n == 1 or (w / w.sum() * np.abs(each - ref)).max() > 1e-3 * abs(ref)
