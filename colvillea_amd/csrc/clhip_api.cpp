@@ -132,6 +132,7 @@ struct clhip_ctx
     uint64_t                 blas_builds = 0; /* mesh trees built since creation */
     bool                     have_blas = false, have_tlas = false;
     DevBuf                   d_nodes, d_tris, d_meshes, d_shade, d_tan, d_idx, d_inst;
+    DevBuf                   d_pos, d_nrm, d_uv; /* read by the shading records' build only; kept for the next */
     size_t                   node_bytes = 0, tri_bytes = 0; /* in use in d_nodes, d_tris */
     uint2*                   noalloc_stack = nullptr; /* this device's scratch of clhip_trace_rays_device */
     std::vector<InstanceRec> inst;
@@ -1451,18 +1452,15 @@ static int assemble_blas(clhip_ctx* ctx)
     CLHIP_CHECK(ctx, upload(ctx->d_meshes, recs));
     CLHIP_CHECK(ctx, upload(ctx->d_tan, tan));
     CLHIP_CHECK(ctx, upload(ctx->d_idx, idx));
-    {
-        DevBuf d_pos, d_nrm, d_uv; /* read by the shading records' build only */
-        CLHIP_CHECK(ctx, upload(d_pos, pos));
-        CLHIP_CHECK(ctx, upload(d_nrm, nrm));
-        CLHIP_CHECK(ctx, upload(d_uv, uv));
-        CLHIP_CHECK(ctx, ctx->d_shade.alloc(std::max<size_t>(tris.size() * sizeof(ShadeRec), 16)));
-        for (const MeshRec& me : recs)
-            CLHIP_CHECK(ctx, clpt::launch_shade_recs(ctx->stream, me, ctx->d_idx.as<const uint32_t>(), d_pos.as<const float>(),
-                                                     d_nrm.as<const float>(), d_uv.as<const float>(),
-                                                     ctx->d_shade.as<ShadeRec>()));
-        CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    }
+    CLHIP_CHECK(ctx, upload(ctx->d_pos, pos));
+    CLHIP_CHECK(ctx, upload(ctx->d_nrm, nrm));
+    CLHIP_CHECK(ctx, upload(ctx->d_uv, uv));
+    CLHIP_CHECK(ctx, ctx->d_shade.alloc(std::max<size_t>(tris.size() * sizeof(ShadeRec), 16)));
+    CLHIP_CHECK(ctx, clpt::launch_shade_recs(ctx->stream, ctx->d_meshes.as<const MeshRec>(), (uint32_t)recs.size(),
+                                             (uint32_t)tris.size(), ctx->d_idx.as<const uint32_t>(),
+                                             ctx->d_pos.as<const float>(), ctx->d_nrm.as<const float>(),
+                                             ctx->d_uv.as<const float>(), ctx->d_shade.as<ShadeRec>()));
+    CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
     ctx->blas_nodes4 = std::move(nodes4);
     ctx->blas_nodes8 = std::move(nodes8);
     ctx->meshes      = std::move(infos);

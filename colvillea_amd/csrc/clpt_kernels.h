@@ -41,9 +41,10 @@ hipError_t launch_sum_waves(hipStream_t s, const WaveCounts& wc, uint32_t rows, 
 hipError_t launch_resolve(hipStream_t s, const double* accum, uint32_t npix, uint32_t spp, int srgb, float4* out);
 hipError_t launch_srgb_batch(hipStream_t s, const float* in, uint32_t n, int decode, float* out);
 hipError_t launch_texture_u8(hipStream_t s, const uchar4* in, uint32_t n, int srgb, float4* out);
-/* The shading records of one mesh from the shared indexed arrays. */
-hipError_t launch_shade_recs(hipStream_t s, const MeshRec& me, const uint32_t* idx, const float* pos, const float* nrm,
-                             const float* uv, ShadeRec* out);
+/* The shading records of every mesh's triangles from the shared indexed
+ * arrays. */
+hipError_t launch_shade_recs(hipStream_t s, const MeshRec* meshes, uint32_t nmeshes, uint32_t ntris, const uint32_t* idx,
+                             const float* pos, const float* nrm, const float* uv, ShadeRec* out);
 /* The traversal form of n BVH4 nodes. */
 hipError_t launch_pack_nodes(hipStream_t s, const Node4* in, uint32_t n, Node4P* out);
 hipError_t launch_dome_tables(hipStream_t s, const float4* tex, uint32_t w, uint32_t h, float* pcond, float* cdfcond,

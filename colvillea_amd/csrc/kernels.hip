@@ -1877,19 +1877,32 @@ __global__ __launch_bounds__(256) void k_dome_cuts(uint32_t w, uint32_t h, const
 
 /* ------------------------------------------------------------ scene packing */
 
-/* The shading records of one mesh, a thread per triangle. */
-__global__ __launch_bounds__(256) void k_shade_recs(MeshRec me, const uint32_t* __restrict__ idx, const float* __restrict__ pos,
+/* The shading records of all meshes in one launch, a thread per triangle; its
+ * mesh is the last whose triangles begin at or before it (meshes lie in
+ * order; an empty one begins where the next does).  A launch per mesh took 10
+ * ms for 4000 meshes of 12 triangles. */
+__global__ __launch_bounds__(256) void k_shade_recs(const MeshRec* __restrict__ meshes, uint32_t nmeshes, uint32_t ntris,
+                                                    const uint32_t* __restrict__ idx, const float* __restrict__ pos,
                                                     const float* __restrict__ nrm, const float* __restrict__ uv,
                                                     ShadeRec* __restrict__ out)
 {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= me.ntris)
+    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= ntris)
         return;
-    const size_t g = (size_t)me.idx_off + t;
+    uint32_t lo = 0, hi = nmeshes; /* meshes[lo] begins at or before g, meshes[hi] after it */
+    while (hi - lo > 1u)
+    {
+        const uint32_t mid = (lo + hi) / 2u;
+        if (meshes[mid].idx_off <= g)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    const MeshRec me = meshes[lo];
     ShadeRec     r{};
     for (int k = 0; k < 3; ++k)
     {
-        const size_t v = (size_t)idx[3 * g + k] + me.vtx_off;
+        const size_t v = (size_t)idx[3 * (size_t)g + k] + me.vtx_off;
         for (int a = 0; a < 3; ++a)
         {
             r.p[k][a] = pos[3 * v + a];
@@ -2237,11 +2250,12 @@ hipError_t launch_texture_u8(hipStream_t s, const uchar4* in, uint32_t n, int sr
     return hipGetLastError();
 }
 
-hipError_t launch_shade_recs(hipStream_t s, const MeshRec& me, const uint32_t* idx, const float* pos, const float* nrm,
-                             const float* uv, ShadeRec* out)
+hipError_t launch_shade_recs(hipStream_t s, const MeshRec* meshes, uint32_t nmeshes, uint32_t ntris, const uint32_t* idx,
+                             const float* pos, const float* nrm, const float* uv, ShadeRec* out)
 {
-    if (me.ntris)
-        hipLaunchKernelGGL(k_shade_recs, dim3((me.ntris + 255u) / 256u), dim3(256), 0, s, me, idx, pos, nrm, uv, out);
+    if (ntris)
+        hipLaunchKernelGGL(k_shade_recs, dim3((ntris + 255u) / 256u), dim3(256), 0, s, meshes, nmeshes, ntris, idx, pos, nrm,
+                           uv, out);
     return hipGetLastError();
 }
 
