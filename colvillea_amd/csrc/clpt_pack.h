@@ -12,30 +12,24 @@
 
 /* The largest half not above x, as its bits: 10 bits of fraction, exponents
  * -14..15 (no subnormals: values in (-2^-14, 2^-14) go to -2^-14 or 0), and
- * -inf below the half range.  Values above it give the largest half. */
+ * -inf below the half range and for NaN.  Values above it give the largest
+ * half. */
 __host__ __device__ inline uint16_t half_floor(double x)
 {
-    const double tiny = 6.103515625e-05; /* 2^-14 */
-    if (x >= 0.0 && x < tiny)
-        return 0u;
-    if (x < 0.0 && x > -tiny)
-        return (uint16_t)(0x8000u | (1u << 10));
+    if (!(x >= -65504.0))
+        return 0xfc00u;
     if (x >= 65504.0)
         return 0x7bffu;
-    if (x < -65504.0)
-        return 0xfc00u;
-    int          e;
-    const double f = frexp(fabs(x), &e);    /* |x| = f 2^e, f in [1/2, 1) */
-    const double m = f * 2048.0;            /* 11 significant bits: [1024, 2048) */
-    uint32_t     k = (uint32_t)m;           /* towards zero */
-    if (x < 0.0 && (double)k != m)
-        ++k;                                /* away from zero */
-    if (k == 2048u)
-    {
-        k = 1024u;
-        ++e;
-    }
-    return (uint16_t)((x < 0.0 ? 0x8000u : 0u) | ((uint32_t)(e + 14) << 10) | (k - 1024u));
+    if (fabs(x) < 6.103515625e-05) /* 2^-14 */
+        return x < 0.0 ? 0x8400u : 0u;
+    uint64_t b;
+    memcpy(&b, &x, sizeof(b));
+    /* truncated towards zero; a negative value with a remainder is the next
+     * one away from it, a carry out of the fraction the next exponent */
+    uint32_t h = ((uint32_t)(b >> 52 & 0x7ffu) - 1008u) << 10 | (uint32_t)(b >> 42 & 0x3ffu);
+    if (b >> 63 && (b & ((1ull << 42) - 1u)))
+        ++h;
+    return (uint16_t)((uint32_t)(b >> 63) << 15 | h);
 }
 __host__ __device__ inline uint16_t half_ceil(double x) { return (uint16_t)(half_floor(-x) ^ 0x8000u); }
 
@@ -47,29 +41,36 @@ __host__ __device__ inline void pack_node4(const Node4& in, Node4P& out)
     double       ext   = 0.0;
     for (int a = 0; a < 3; ++a)
     {
+        /* over the planes that are finite; the others pack to infinities */
         float l = INFINITY, h = -INFINITY;
         for (int c = 0; c < 4; ++c)
-            if (in.child[c] != CLPT_CHILD_EMPTY)
+            for (int k = 0; k < 2; ++k)
             {
-                l = fminf(l, lo[a][c]);
-                h = fmaxf(h, hi[a][c]);
+                const float x = k ? hi[a][c] : lo[a][c];
+                if (in.child[c] != CLPT_CHILD_EMPTY && fabsf(x) < INFINITY)
+                {
+                    l = fminf(l, x);
+                    h = fmaxf(h, x);
+                }
             }
-        if (l <= h && l >= -3.0e38f && h <= 3.0e38f)
+        if (l <= h)
         {
             p[a] = l;
             ext  = fmax(ext, (double)h - (double)l);
         }
     }
-    /* s = 2^k with the extent at most 2^14 s; far out of range, planes
-     * beyond the halves become infinite */
+    /* s = 2^k with the extent at most 2^14 s */
     int k = -60;
     if (ext > 0.0)
     {
         (void)frexp(ext, &k); /* ext < 2^k */
         k -= 14;
-        k = k < -60 ? -60 : (k > 60 ? 60 : k);
+        k = k < -60 ? -60 : k;
     }
-    const double s = ldexp(1.0, k), w = ext * 9.5367431640625e-07; /* 2^-20 */
+    /* From 2^60 on, (p - o) inv can overflow (|inv| is at most 1e20) for a
+     * ray that lies in a child's box: such boxes take every ray. */
+    const bool   open = ext >= 1.152921504606847e18;
+    const double r = ldexp(1.0, -k), w = ext * 9.5367431640625e-07; /* 2^-20 */
     for (int a = 0; a < 3; ++a)
         for (int c = 0; c < 4; ++c)
         {
@@ -79,12 +80,12 @@ __host__ __device__ inline void pack_node4(const Node4& in, Node4P& out)
                 out.pl[a][1][c] = 0xfc00u; /* -inf */
                 continue;
             }
-            out.pl[a][0][c] = half_floor(((double)lo[a][c] - w - (double)p[a]) / s);
-            out.pl[a][1][c] = half_ceil(((double)hi[a][c] + w - (double)p[a]) / s);
+            out.pl[a][0][c] = open ? 0xfc00u : half_floor(((double)lo[a][c] - w - (double)p[a]) * r);
+            out.pl[a][1][c] = open ? 0x7c00u : half_ceil(((double)hi[a][c] + w - (double)p[a]) * r);
         }
     for (int a = 0; a < 3; ++a)
         out.p[a] = p[a];
-    out.s = (float)s;
+    out.s = open ? 1.0f : (float)ldexp(1.0, k);
     for (int c = 0; c < 4; ++c)
         out.child[c] = in.child[c];
 }

@@ -27,7 +27,9 @@ static_assert(sizeof(Node4) == 128, "Node4 is two 64-byte halves");
  * (pack_node4).  A child's planes on axis a are p[a] + q s, q a half float
  * rounded outward after the box was widened by 2^-20 of the node's extent,
  * which covers the rounding of the slab test's arithmetic on them: a packed
- * box culls nothing that the float box keeps, so hits are the same bits.
+ * box culls nothing that the float box keeps, so hits are the same bits
+ * (checked for directions of length 1e-20 to 1e20 and extents of 1e-30 to
+ * 1e37; boxes of nodes of 2^60 and more take every ray).
  * Empty slots hold an inverted infinite box. ---- */
 struct alignas(16) Node4P
 {

@@ -1,6 +1,7 @@
 /* Host check of the packed BVH4 node (colvillea_amd/csrc/clpt_pack.h): over
- * nodes of many extents and places (flat, tiny, huge, far from the origin,
- * with empty slots), every packed box contains the float box, empty slots
+ * nodes of many extents and places (flat, tiny, huge beyond what halves and
+ * the slab test's products hold, far from the origin, with planes that are
+ * not finite, with empty slots), every packed box contains the float box, empty slots
  * are inverted and infinite, and the packed slab test passes every child
  * that the float slab test passes, for rays that graze and miss boxes,
  * start inside, far away and along axes.  Prints "ok" or the failures. */
@@ -63,8 +64,8 @@ int main()
 {
     std::mt19937                           rng(7);
     std::uniform_real_distribution<double> U(-1.0, 1.0);
-    const double sizes[]  = {1e-12, 1e-6, 1e-3, 0.03, 1.0, 40.0, 1e5, 1e12};
-    const double places[] = {0.0, 1e-4, 1.0, 30.0, 1e4, 1e9};
+    const double sizes[]  = {1e-30, 1e-12, 1e-6, 1e-3, 0.03, 1.0, 40.0, 1e5, 1e12, 1e21, 1e25, 1e37};
+    const double places[] = {0.0, 1e-4, 1.0, 30.0, 1e4, 1e9, 1e22};
     long         passes = 0, both = 0;
     for (double size : sizes)
         for (double place : places)
@@ -88,6 +89,17 @@ int main()
                         hi[a][c] = c < 4 - empties ? (float)std::fmax(u, v) : -INFINITY;
                     }
                 }
+                /* boxes of vertices that are not finite */
+                const int odd = it % 10, oa = it / 10 % 3;
+                if (odd == 7)
+                    hi[oa][0] = INFINITY;
+                if (odd == 8)
+                {
+                    lo[oa][0] = -INFINITY;
+                    hi[oa][0] = INFINITY;
+                }
+                if (odd == 9)
+                    (it % 4 < 2 ? lo : hi)[oa][0] = NAN;
                 Node4P p;
                 pack_node4(nd, p);
                 for (int c = 0; c < 4; ++c)
@@ -100,7 +112,7 @@ int main()
                             if (!(l == INFINITY && h == -INFINITY))
                                 fail("empty slot", l, h);
                         }
-                        else if (!(l <= lo[a][c] && h >= hi[a][c]))
+                        else if (l > lo[a][c] || h < hi[a][c] || l != l || h != h)
                             fail("box", l - lo[a][c], hi[a][c] - h);
                     }
                 for (int r = 0; r < 200; ++r)
@@ -120,11 +132,13 @@ int main()
                             d[a] = 0.0f;
                     }
                     const double len = std::sqrt((double)d[0] * d[0] + (double)d[1] * d[1] + (double)d[2] * d[2]);
-                    if (!(len > 0.0))
+                    if (!(len > 0.0 && len < INFINITY))
                         continue;
+                    /* half of the rays are not of unit length, as inside a scaled instance */
+                    const double mag = r % 4 < 2 ? 1.0 : std::pow(10.0, 20.0 * U(rng));
                     for (int a = 0; a < 3; ++a)
                     {
-                        d[a]   = (float)(d[a] / len);
+                        d[a]   = (float)(d[a] / len * mag);
                         inv[a] = rcp(d[a]);
                     }
                     const float tmin = r % 2 ? 0.001f : 0.0f, tmax = r % 3 ? 3.402823466e+38f : (float)len;

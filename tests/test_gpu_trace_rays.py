@@ -10,6 +10,7 @@ import pytest
 
 from colvillea_amd import Integrator, IntegratorType, scenes, upload_scene
 from colvillea_amd import _capi as capi
+from colvillea_amd.integrator import TriangleMesh
 from test_zz_no_alloc import rays, trace_device
 
 pytestmark = pytest.mark.gpu
@@ -40,3 +41,21 @@ def test_results_do_not_depend_on_the_batch(width):
                 capi.check(capi.lib().clhip_occlusion_batch(integ.ctx, capi.fptr(r), n,
                                                             occ.ctypes.data_as(C.POINTER(C.c_uint8))), integ.ctx)
                 assert np.array_equal(occ != 0, hit[:, 0] != 0)
+
+
+@pytest.mark.parametrize("width", [4, 8], ids=["bvh4", "bvh8"])
+@pytest.mark.parametrize("far", [1e3, 1e12, 1e19, 1e21])
+def test_a_near_triangle_beside_a_far_one(width, far):
+    """Both lie in one node, whose extent is up to 1e21: rays along the axes
+    (reciprocals up to 1e20) through the near one still hit it."""
+    near = np.array([[-1, -1, -5], [3, -1, -5], [-1, 3, -5]], np.float32)
+    v = np.concatenate([near, near + np.float32([-far, 0, 0]), near + np.float32([0, -far, 0])]).astype(np.float32)
+    mesh = TriangleMesh(v, np.arange(9, dtype=np.uint32).reshape(3, 3))
+    r = np.array([[0.25 * i, 0.25 * j, 0, 0, 0, 0, -1, 3e38] for i in range(3) for j in range(3)], np.float32)
+    with Integrator.createIntegrator(IntegratorType.WavefrontPathTracing, 8, 8) as integ:
+        integ.setBVHWidth(width)
+        integ.buildBLAS([mesh])
+        integ.buildTLAS([mesh], [0])
+        for any_hit in (False, True):
+            hit, prim = trace_device(integ, r, any_hit)
+            assert np.all(hit[:, 0] == (1.0 if any_hit else 5.0)) and np.all(prim == 0), (hit, prim)
