@@ -7,6 +7,7 @@
 #include "bvh_build.h"
 #include "clpt_guide.h"
 #include "clpt_kernels.h"
+#include "clpt_pack.h"
 #include "host_copy.h"
 
 #include <hip/hip_runtime.h>
@@ -134,6 +135,8 @@ struct clhip_ctx
     DevBuf                   d_nodes, d_tris, d_meshes, d_shade, d_tan, d_idx, d_inst;
     DevBuf                   d_pos, d_nrm, d_uv; /* read by the shading records' build only; kept for the next */
     size_t                   node_bytes = 0, tri_bytes = 0; /* in use in d_nodes, d_tris */
+    DevBuf                   d_nodes_raw; /* BVH4 nodes on their way into d_nodes */
+    bool                     mesh_nodes_packed = false; /* d_nodes begins with blas_nodes4, packed */
     uint2*                   noalloc_stack = nullptr; /* this device's scratch of clhip_trace_rays_device */
     std::vector<InstanceRec> inst;
     std::vector<uint32_t>    inst_entity;
@@ -1027,6 +1030,9 @@ struct Tmp
  * BVH8 the decoded box, which contains the subtree). */
 constexpr size_t kRebraidParts = 64;
 
+/* BVH4 nodes packed at a time (4 MiB of float nodes) */
+constexpr size_t kPackNodes = 32768;
+
 struct TopPrim
 {
     uint32_t ref;
@@ -1460,7 +1466,7 @@ static int assemble_blas(clhip_ctx* ctx)
                                              (uint32_t)tris.size(), ctx->d_idx.as<const uint32_t>(),
                                              ctx->d_pos.as<const float>(), ctx->d_nrm.as<const float>(),
                                              ctx->d_uv.as<const float>(), ctx->d_shade.as<ShadeRec>()));
-    CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    ctx->mesh_nodes_packed = false;
     ctx->blas_nodes4 = std::move(nodes4);
     ctx->blas_nodes8 = std::move(nodes8);
     ctx->meshes      = std::move(infos);
@@ -1631,10 +1637,14 @@ int clhip_build_tlas(clhip_ctx* ctx, const uint32_t* mesh_of_instance, const uin
     if (need > 128u)
         return fail(ctx, CLHIP_E_UNSUPPORTED, "tree too deep for the traversal stack (TLAS %u + BLAS %u levels)",
                     r.max_depth, max_blas_depth);
-    /* traversal addresses nodes by 32-bit byte offsets */
+    /* traversal addresses nodes by 32-bit byte offsets (BVH4 trees are
+     * counted as built, 128 bytes a node; packed they are smaller) */
     const size_t nbytes = ctx->bvh_width == 8 ? nodes8.size() * sizeof(Node8) : nodes4.size() * sizeof(Node4);
     if (nbytes > 0xffffffffull)
         return fail(ctx, CLHIP_E_UNSUPPORTED, "node array of %zu bytes exceeds 4 GiB", nbytes);
+    /* the records go up now, so traversal alone (clhip_trace_rays_device)
+     * needs no further upload; sync_instances fills in the materials */
+    CLHIP_CHECK(ctx, upload(ctx->d_inst, inst));
     if (ctx->bvh_width == 8)
     {
         CLHIP_CHECK(ctx, upload(ctx->d_nodes, nodes8));
@@ -1642,18 +1652,34 @@ int clhip_build_tlas(clhip_ctx* ctx, const uint32_t* mesh_of_instance, const uin
     }
     else
     {
-        /* uploaded as built and packed on the device */
-        Tmp raw;
-        CLHIP_CHECK(ctx, raw.from_host(nodes4.data(), nodes4.size()));
-        CLHIP_CHECK(ctx, ctx->d_nodes.alloc(std::max<size_t>(nodes4.size() * sizeof(Node4P), 16)));
-        CLHIP_CHECK(ctx, clpt::launch_pack_nodes(ctx->stream, raw.b.as<const Node4>(), (uint32_t)nodes4.size(),
-                                                 ctx->d_nodes.as<Node4P>()));
-        CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+        /* The meshes' nodes come first and stay as they are until the BLAS is
+         * built again: they are sent as built, a piece at a time, and packed
+         * on the device, once.  The top tree's few are packed here, so moving
+         * an instance costs no launch and sends 80 bytes a node. */
+        const size_t bytes = std::max<size_t>(nodes4.size() * sizeof(Node4P), 16), mesh = ctx->blas_nodes4.size();
+        if (bytes > ctx->d_nodes.bytes)
+            ctx->mesh_nodes_packed = false; /* about to move */
+        CLHIP_CHECK(ctx, ctx->d_nodes.alloc(bytes));
+        if (!ctx->mesh_nodes_packed)
+        {
+            CLHIP_CHECK(ctx, ctx->d_nodes_raw.alloc(std::min(mesh, kPackNodes) * sizeof(Node4)));
+            for (size_t at = 0; at < mesh; at += kPackNodes)
+            {
+                const size_t n = std::min(mesh - at, kPackNodes);
+                CLHIP_CHECK(ctx, ctx->copier->from_host(ctx->stream, ctx->d_nodes_raw.p, nodes4.data() + at, n * sizeof(Node4)));
+                CLHIP_CHECK(ctx, clpt::launch_pack_nodes(ctx->stream, ctx->d_nodes_raw.as<const Node4>(), (uint32_t)n,
+                                                         ctx->d_nodes.as<Node4P>() + at));
+            }
+            ctx->mesh_nodes_packed = true;
+        }
+        std::vector<Node4P> top(nodes4.size() - mesh);
+        for (size_t k = 0; k < top.size(); ++k)
+            pack_node4(nodes4[mesh + k], top[k]);
+        if (!top.empty())
+            CLHIP_CHECK(ctx, hipMemcpy(ctx->d_nodes.as<Node4P>() + mesh, top.data(), top.size() * sizeof(Node4P),
+                                       hipMemcpyHostToDevice));
         ctx->node_bytes = nodes4.size() * sizeof(Node4P);
     }
-    /* the records go up now, so traversal alone (clhip_trace_rays_device)
-     * needs no further upload; sync_instances fills in the materials */
-    CLHIP_CHECK(ctx, upload(ctx->d_inst, inst));
     ctx->inst        = std::move(inst);
     ctx->inst_entity = std::move(ent);
     ctx->tlas_root   = r.root;

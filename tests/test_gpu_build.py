@@ -7,7 +7,8 @@ import pytest
 
 import orc
 from colvillea_amd import Integrator, IntegratorType, scenes, upload_scene
-from colvillea_amd.integrator import TriangleMesh
+from colvillea_amd import _capi as capi
+from colvillea_amd.integrator import DiffuseMtl, Entity, TriangleMesh
 from test_gpu_edges import _gpu_tables
 
 pytestmark = pytest.mark.gpu
@@ -87,3 +88,56 @@ def test_rebuild_after_an_edit(width):
             integ.buildTLAS([d.meshes[m] for m in d.instance_mesh], list(range(len(d.instance_mesh))), d.instance_xform)
             sums, cnt = _render(integ, d)
             _check(d, sums, cnt, _gpu_tables(integ, d))
+
+
+def _hits(integ, rays):
+    n = len(rays)
+    t, b, inst, prim = np.zeros(n, np.float32), np.zeros((n, 2), np.float32), np.zeros(n, np.uint32), np.zeros(n, np.uint32)
+    capi.check(capi.lib().clhip_trace_batch(integ.ctx, capi.fptr(rays), n, capi.fptr(t), capi.fptr(b), capi.uptr(inst),
+                                            capi.uptr(prim)), integ.ctx)
+    return t, b, inst, prim
+
+
+def test_packed_nodes_of_large_trees_and_of_moved_instances():
+    """Trees of more nodes than are packed at a time: hits equal those of
+    the other tree width (which is not packed), for a first build, moved
+    instances, more instances (the node array grows) and fewer."""
+    side = 301
+    g = np.linspace(-4.0, 4.0, side, dtype=np.float32)
+    x, z = np.meshgrid(g, g, indexing="ij")
+    y = (0.3 * np.sin(3.0 * x) * np.cos(2.0 * z)).astype(np.float32)
+    i = np.arange((side - 1) * side).reshape(side - 1, side)[:, :-1].ravel()
+    tri = np.concatenate([np.stack([i, i + 1, i + side], 1), np.stack([i + 1, i + side + 1, i + side], 1)]).astype(np.uint32)
+    mesh = TriangleMesh(np.stack([x.ravel(), y.ravel(), z.ravel()], 1), tri)
+    ball = scenes.icosphere(2)
+    rng = np.random.default_rng(3)
+    n = 50000
+    o = rng.uniform(-5.0, 5.0, (n, 3))
+    d = rng.uniform(-6.0, 6.0, (n, 3)) * [1.0, 0.1, 1.0] - o  # a third aim past the terrain
+    rays = np.concatenate([o, np.zeros((n, 1)), d / np.linalg.norm(d, axis=1, keepdims=True), np.full((n, 1), 3e38)],
+                          1).astype(np.float32)
+    ctx = []
+    for width in (4, 8):
+        integ = Integrator.createIntegrator(IntegratorType.WavefrontPathTracing, 8, 8)
+        integ.setBVHWidth(width)
+        integ.buildMaterials([DiffuseMtl((0.5, 0.5, 0.5))])
+        integ.buildGeometryEntities([Entity(0)] * 71)
+        integ.buildBLAS([mesh, ball])
+        ctx.append(integ)
+    try:
+        for balls, seed in ((1, 0), (1, 1), (70, 2), (3, 3), (70, 4)):
+            r = np.random.default_rng(seed)
+            xf = np.concatenate([scenes.IDENTITY[None]] + [scenes.translate_scale(r.uniform(-3, 3, 3), r.uniform(0.1, 0.6))[None]
+                                                           for _ in range(balls)]).astype(np.float32)
+            out = []
+            for integ in ctx:
+                integ.buildTLAS([mesh] + [ball] * balls, list(range(balls + 1)), xf)
+                out.append(_hits(integ, rays))
+            assert 0.2 < (out[0][0] > 0).mean() < 0.95 and np.any(out[0][2] == balls)
+            for a, b in zip(*out):
+                assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), (balls, seed)
+        nodes = (ctx[0].counters()["scene_bytes"] - 48 * (len(tri) + len(ball.triangles))) // 80
+        assert nodes > 32768, nodes
+    finally:
+        for integ in ctx:
+            integ.close()
