@@ -1453,6 +1453,10 @@ static int assemble_blas(clhip_ctx* ctx)
         idx.insert(idx.end(), mb.idx.begin(), mb.idx.end());
     }
     CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream)); /* the old arrays may be in use */
+    /* a failure from here on leaves no mesh that a trace may follow */
+    ctx->have_blas         = false;
+    ctx->have_tlas         = false;
+    ctx->mesh_nodes_packed = false;
     CLHIP_CHECK(ctx, upload(ctx->d_tris, tris));
     ctx->tri_bytes = tris.size() * sizeof(TriRec);
     CLHIP_CHECK(ctx, upload(ctx->d_meshes, recs));
@@ -1466,13 +1470,11 @@ static int assemble_blas(clhip_ctx* ctx)
                                              (uint32_t)tris.size(), ctx->d_idx.as<const uint32_t>(),
                                              ctx->d_pos.as<const float>(), ctx->d_nrm.as<const float>(),
                                              ctx->d_uv.as<const float>(), ctx->d_shade.as<ShadeRec>()));
-    ctx->mesh_nodes_packed = false;
     ctx->blas_nodes4 = std::move(nodes4);
     ctx->blas_nodes8 = std::move(nodes8);
     ctx->meshes      = std::move(infos);
     ctx->mesh_recs   = std::move(recs);
-    ctx->have_blas   = true;
-    ctx->have_tlas   = false; /* roots moved: the TLAS must be rebuilt */
+    ctx->have_blas   = true; /* the roots moved: the TLAS must be rebuilt */
     return CLHIP_OK;
 }
 
@@ -1642,6 +1644,7 @@ int clhip_build_tlas(clhip_ctx* ctx, const uint32_t* mesh_of_instance, const uin
     const size_t nbytes = ctx->bvh_width == 8 ? nodes8.size() * sizeof(Node8) : nodes4.size() * sizeof(Node4);
     if (nbytes > 0xffffffffull)
         return fail(ctx, CLHIP_E_UNSUPPORTED, "node array of %zu bytes exceeds 4 GiB", nbytes);
+    ctx->have_tlas = false; /* until all of it is in place */
     /* the records go up now, so traversal alone (clhip_trace_rays_device)
      * needs no further upload; sync_instances fills in the materials */
     CLHIP_CHECK(ctx, upload(ctx->d_inst, inst));
