@@ -59,3 +59,32 @@ def test_a_near_triangle_beside_a_far_one(width, far):
         for any_hit in (False, True):
             hit, prim = trace_device(integ, r, any_hit)
             assert np.all(hit[:, 0] == (1.0 if any_hit else 5.0)) and np.all(prim == 0), (hit, prim)
+
+
+@pytest.mark.parametrize("width", [4, 8], ids=["bvh4", "bvh8"])
+def test_rays_without_a_place_or_direction_miss(width):
+    """NaN in a ray lets it into every box, also the empty slots' (they hold
+    no reference): it misses, and the rays beside it keep their hits."""
+    ball = scenes.icosphere(1)
+    xf = np.stack([scenes.IDENTITY, scenes.translate_scale((2.5, 0.0, 0.0), 0.7), scenes.translate_scale((0.0, 2.5, 0.0), 0.4)])
+    rng = np.random.default_rng(2)
+    n = 192
+    o = rng.uniform(-4.0, 4.0, (n, 3))
+    d = rng.uniform(-1.0, 1.0, (n, 3)) + [[0.8, 0.8, 0.0]] - o
+    good = np.concatenate([o, np.zeros((n, 1)), d / np.linalg.norm(d, axis=1, keepdims=True), np.full((n, 1), 3e38)],
+                          1).astype(np.float32)
+    bad = good.copy()
+    at = np.arange(0, n, 3)
+    for i, k in enumerate(at):
+        bad[k, [[0], [0, 1, 2], [4], [4, 5, 6], [0, 1, 2, 4, 5, 6]][i % 5]] = np.nan if i % 2 else np.inf
+    with Integrator.createIntegrator(IntegratorType.WavefrontPathTracing, 8, 8) as integ:
+        integ.setBVHWidth(width)
+        integ.buildBLAS([ball])
+        integ.buildTLAS([ball] * 3, [0, 1, 2], xf.astype(np.float32))
+        for any_hit in (False, True):
+            ref, ref_prim = trace_device(integ, good, any_hit)
+            hit, prim = trace_device(integ, bad, any_hit)
+            rest = np.setdiff1d(np.arange(n), at)
+            assert np.array_equal(hit[rest].view(np.uint32), ref[rest].view(np.uint32)) and (ref[rest, 0] > 0).sum() > 20
+            assert np.array_equal(prim[rest], ref_prim[rest])
+            assert np.all(hit[at, 0] == (0.0 if any_hit else -1.0)), hit[at, 0]
