@@ -90,4 +90,40 @@ __host__ __device__ inline void pack_node4(const Node4& in, Node4P& out)
         out.child[c] = in.child[c];
 }
 
+/* The slab test on packed planes.  On each axis the plane of half q lies at
+ * p + q s, at the ray's t = q (s inv) + (p - o) inv, one fused multiply-add:
+ * the ray in the node's units is (i, b) = (s inv, (p - o) inv). */
+struct PackRay
+{
+    float bx, ix, by, iy, bz, iz;
+};
+
+__host__ __device__ inline PackRay pack_ray(float px, float py, float pz, float s, float ox, float oy, float oz, float invx,
+                                            float invy, float invz)
+{
+    PackRay r;
+    r.bx = (px - ox) * invx;
+    r.ix = s * invx;
+    r.by = (py - oy) * invy;
+    r.iy = s * invy;
+    r.bz = (pz - oz) * invz;
+    r.iz = s * invz;
+    return r;
+}
+
+/* A child by its near and far planes (lo and hi by the sign of inv): the
+ * entry distance, padded by 2e-5 relative (all on the near side), and whether
+ * the ray meets the box in [tmin, tmax].  An empty slot (inverted infinite
+ * box) gives +inf > far, but where every slab overflows to NaN. */
+__host__ __device__ inline bool pack_slab(const PackRay& r, float nx, float ny, float nz, float fx, float fy, float fz,
+                                          float tmin, float tmax, float& tnear)
+{
+    const float tnx = __builtin_fmaf(nx, r.ix, r.bx), tfx = __builtin_fmaf(fx, r.ix, r.bx);
+    const float tny = __builtin_fmaf(ny, r.iy, r.by), tfy = __builtin_fmaf(fy, r.iy, r.by);
+    const float tnz = __builtin_fmaf(nz, r.iz, r.bz), tfz = __builtin_fmaf(fz, r.iz, r.bz);
+    tnear             = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, tmin)) * 0.99998f;
+    const float tfar  = fminf(fminf(tfx, tfy), fminf(tfz, tmax));
+    return tnear <= tfar;
+}
+
 #endif

@@ -217,27 +217,17 @@ __device__ __forceinline__ bool visit_node<4>(const SceneView& sc, const RayW& r
     const uint32_t nx[2] = {gx ? px.z : px.x, gx ? px.w : px.y}, fx[2] = {gx ? px.x : px.z, gx ? px.y : px.w};
     const uint32_t ny[2] = {gy ? py.z : py.x, gy ? py.w : py.y}, fy[2] = {gy ? py.x : py.z, gy ? py.y : py.w};
     const uint32_t nz[2] = {gz ? pz.z : pz.x, gz ? pz.w : pz.y}, fz[2] = {gz ? pz.x : pz.z, gz ? pz.y : pz.w};
-    /* the ray in the node's units, and a plane's distance as one fused
-     * multiply-add of its half: t = q (s inv) + (p - o) inv */
-    const float s_ = __uint_as_float(ps.w);
-    const float bx = (__uint_as_float(ps.x) - r.o.x) * r.inv.x, ix = s_ * r.inv.x;
-    const float by = (__uint_as_float(ps.y) - r.o.y) * r.inv.y, iy = s_ * r.inv.y;
-    const float bz = (__uint_as_float(ps.z) - r.o.z) * r.inv.z, iz = s_ * r.inv.z;
-    float       tn[4];
-    uint32_t    cr[4] = {ch.x, ch.y, ch.z, ch.w};
+    const PackRay  pr = pack_ray(__uint_as_float(ps.x), __uint_as_float(ps.y), __uint_as_float(ps.z), __uint_as_float(ps.w),
+                                 r.o.x, r.o.y, r.o.z, r.inv.x, r.inv.y, r.inv.z);
+    float          tn[4];
+    uint32_t       cr[4] = {ch.x, ch.y, ch.z, ch.w};
 #pragma unroll
     for (int c = 0; c < 4; ++c)
     {
-        const auto  q   = [c](const uint32_t* w) { return (float)__builtin_bit_cast(h2v, w[c >> 1])[c & 1]; };
-        const float tnx = __builtin_fmaf(q(nx), ix, bx), tfx = __builtin_fmaf(q(fx), ix, bx);
-        const float tny = __builtin_fmaf(q(ny), iy, by), tfy = __builtin_fmaf(q(fy), iy, by);
-        const float tnz = __builtin_fmaf(q(nz), iz, bz), tfz = __builtin_fmaf(q(fz), iz, bz);
-        /* padded by 2e-5 relative, all on the near side */
-        const float tnear = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, tmin)) * 0.99998f;
-        const float tfar  = fminf(fminf(tfx, tfy), fminf(tfz, tmax));
-        /* an empty slot (inverted infinite box) gives tnear = +inf > tfar,
-         * but where every slab overflows to NaN; step() drops its reference */
-        tn[c]             = tnear <= tfar ? tnear : CLPT_FLT_MAX;
+        const auto q = [c](const uint32_t* w) { return (float)__builtin_bit_cast(h2v, w[c >> 1])[c & 1]; };
+        float      tnear;
+        /* where an empty slot's box passes, step() drops its reference */
+        tn[c] = pack_slab(pr, q(nx), q(ny), q(nz), q(fx), q(fy), q(fz), tmin, tmax, tnear) ? tnear : CLPT_FLT_MAX;
     }
     /* nearest first: a 5-comparator sorting network, fixed indices */
     cswap(tn[0], cr[0], tn[1], cr[1]);

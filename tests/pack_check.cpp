@@ -34,7 +34,7 @@ static float rcp(float d)
     return 1.0f / (std::fabs(d) > tiny ? d : (d < 0.0f ? -tiny : tiny));
 }
 
-/* the kernels' slab tests, operation by operation */
+/* the slab test on float boxes (the packed one is the kernels' own) */
 static bool pass_float(const float lo[3], const float hi[3], const float o[3], const float inv[3], float tmin, float tmax)
 {
     float n = tmin, f = tmax;
@@ -49,15 +49,15 @@ static bool pass_float(const float lo[3], const float hi[3], const float o[3], c
 
 static bool pass_packed(const Node4P& p, int c, const float o[3], const float inv[3], float tmin, float tmax)
 {
-    float n = tmin, f = tmax;
+    const PackRay r = pack_ray(p.p[0], p.p[1], p.p[2], p.s, o[0], o[1], o[2], inv[0], inv[1], inv[2]);
+    float         n[3], f[3], t;
     for (int a = 0; a < 3; ++a)
     {
-        const float b = (p.p[a] - o[a]) * inv[a], i = p.s * inv[a];
-        const bool  g = inv[a] < 0.0f;
-        n = std::fmax(n, std::fma((float)half_value(p.pl[a][g ? 1 : 0][c]), i, b));
-        f = std::fmin(f, std::fma((float)half_value(p.pl[a][g ? 0 : 1][c]), i, b));
+        const bool g = inv[a] < 0.0f;
+        n[a]         = (float)half_value(p.pl[a][g ? 1 : 0][c]);
+        f[a]         = (float)half_value(p.pl[a][g ? 0 : 1][c]);
     }
-    return n * 0.99998f <= f;
+    return pack_slab(r, n[0], n[1], n[2], f[0], f[1], f[2], tmin, tmax, t);
 }
 
 int main()
