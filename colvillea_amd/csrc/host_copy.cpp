@@ -52,22 +52,25 @@ bool HostCopier::reserve(size_t bytes)
         return false;
     for (size_t k = 0; k < kSlots; ++k)
         wait_upload(k);
-    const size_t need = std::min(kSlots, (bytes + kPart - 1) / kPart);
+    /* as much of the first slot as is needed, or whole slots */
+    const size_t need = bytes <= kPart ? 1u : std::min(kSlots, (bytes + kPart - 1) / kPart);
+    const size_t room = bytes <= kPart ? (bytes + kPiece - 1) / kPiece * kPiece : need * kPart;
     hipError_t   e    = hipSuccess;
-    bool         fresh = false;
-    if (need > slots_)
+    if (room > room_)
     {
         if (stage_)
             (void)hipHostFree(stage_);
         stage_  = nullptr;
+        room_   = 0;
         slots_  = 0;
         void* p = nullptr;
-        e       = hipHostMalloc(&p, need * kPart, hipHostMallocDefault);
+        e       = hipHostMalloc(&p, room, hipHostMallocDefault);
         if (e == hipSuccess)
         {
-            stage_ = static_cast<char*>(p);
-            slots_ = need;
-            fresh  = true;
+            stage_   = static_cast<char*>(p);
+            room_    = room;
+            slots_   = need;
+            touched_ = false;
         }
     }
     for (size_t k = 0; k < need && e == hipSuccess; ++k)
@@ -79,22 +82,27 @@ bool HostCopier::reserve(size_t bytes)
         if (stage_)
             (void)hipHostFree(stage_);
         stage_   = nullptr;
+        room_    = 0;
         slots_   = 0;
         refused_ = true;
         return false;
     }
-    if (fresh)
-    {
-        /* its pages are mapped as the host first touches them, 100 us and
-         * more per MiB; the stream's work goes on meanwhile */
-        const std::function<void(size_t)> touch = [&](size_t i) {
-            for (size_t at = 0; at < kPiece; at += 4096)
-                *static_cast<volatile char*>(stage_ + i * kPiece + at) = 0;
-        };
-        begin(slots_ * kPer, touch);
-        finish();
-    }
     return true;
+}
+
+/* New staging's pages are mapped as the host first touches them, 100 us and
+ * more per MiB: before a readback waits, while the stream's work goes on. */
+void HostCopier::touch()
+{
+    if (touched_)
+        return;
+    touched_ = true;
+    const std::function<void(size_t)> job = [&](size_t i) {
+        for (size_t at = 0; at < kPiece; at += 4096)
+            *static_cast<volatile char*>(stage_ + i * kPiece + at) = 0;
+    };
+    begin(room_ / kPiece, job);
+    finish();
 }
 
 void HostCopier::work()
@@ -173,6 +181,7 @@ hipError_t HostCopier::to_host(hipStream_t s, void* dst, const void* dev, size_t
         e = hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
+    touch();
     char*        out    = static_cast<char*>(dst);
     const char*  in     = static_cast<const char*>(dev);
     const size_t parts  = (bytes + kPart - 1) / kPart, pieces = (bytes + kPiece - 1) / kPiece;
@@ -239,6 +248,7 @@ hipError_t HostCopier::from_host(hipStream_t s, void* dev, const void* src, size
         e = hipMemcpyAsync(dev, src, bytes, hipMemcpyHostToDevice, s);
         return e == hipSuccess ? hipStreamSynchronize(s) : e; /* src may be reused */
     }
+    touched_ = true; /* the copy into it does */
     const char*  in     = static_cast<const char*>(src);
     char*        out    = static_cast<char*>(dev);
     const size_t parts  = (bytes + kPart - 1) / kPart, pieces = (bytes + kPiece - 1) / kPiece;

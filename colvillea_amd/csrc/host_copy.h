@@ -24,14 +24,14 @@ namespace clpt
  *
  * One HostCopier serves one context (it is not thread-safe).  Its staging and
  * threads are made at the first copy that needs them and kept for the
- * context's life; new pinned memory costs a multiple of what a copy through
- * it does until the host has touched it (100 us and more per MiB with all
- * threads), so there is little of it.  Film of 1920x1080 (31.6 MiB) read back
+ * context's life; the host's first touch of new pinned memory costs 100 us
+ * and more per MiB with all threads, so there is little of it.  Film of 1920x1080 (31.6 MiB) read back
  * after a render, first and later times in a context: 1.9 and 1.9 ms through
  * the runtime, 3.1 and 1.08 with 32 slots of 1 MiB each queued once, 0.89 and
  * 0.85 with these two; two slots of 1 MiB 1.07 later, of 4 MiB or four of 2
- * MiB no faster and up to 1 ms longer the first time.  Below kMin the threads
- * gain nothing: 1.2 MiB takes 97 us either way, 0.3 MiB 39 against 45. */
+ * MiB no faster and up to 1 ms longer the first time.  Below kMin nothing is
+ * gained (0.3 MiB takes 39 us, staged 45); behind a render 1.2 MiB staged is
+ * 13 us sooner than the runtime's, which starts when the render has ended. */
 class HostCopier
 {
 public:
@@ -47,7 +47,7 @@ public:
     hipError_t from_host(hipStream_t s, void* dev, const void* src, size_t bytes);
 
 private:
-    static constexpr size_t   kMin     = 2u << 20;
+    static constexpr size_t   kMin     = 1u << 20;
     static constexpr size_t   kPart    = 2u << 20; /* one transfer, one slot */
     static constexpr size_t   kSlots   = 2;
     static constexpr size_t   kPiece   = 128u << 10; /* what a thread copies at a time */
@@ -56,6 +56,7 @@ private:
 
     /* staging and events for a copy; false: there are none to be had */
     bool reserve(size_t bytes);
+    void touch();
     void wait_upload(size_t k);
     /* job(k) for k = 0..n-1 on the threads from begin() on; the caller's takes
      * those below `end` that are left in help() and all in finish(), which
@@ -66,7 +67,8 @@ private:
     void work();
 
     char*                    stage_ = nullptr;
-    size_t                   slots_ = 0;
+    size_t                   room_ = 0, slots_ = 0;
+    bool                     touched_ = true;
     bool                     refused_ = false; /* pinned memory or an event could not be had */
     hipEvent_t               ev_[kSlots] = {}; /* the last transfer of each slot */
     bool                     up_pending_[kSlots] = {}; /* it was an upload and may not be done */

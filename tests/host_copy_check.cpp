@@ -178,6 +178,7 @@ static constexpr size_t MiB = 1u << 20;
 static std::vector<char> bytes_of(size_t n, uint32_t seed)
 {
     std::vector<char> v(n);
+    v.reserve(n + 1); /* not null for no bytes */
     uint32_t          x = seed * 2654435761u + 1u;
     for (size_t i = 0; i < n; ++i)
     {
@@ -209,7 +210,7 @@ int main(int argc, char** argv)
         {
             /* around pieces, the sizes from which several threads copy, the
              * whole staging and several times it, up and down in turn */
-            for (size_t n : {(size_t)0, (size_t)1, MiB, 2 * MiB - 1, 2 * MiB, 2 * MiB + 1, 5 * MiB / 2, 3 * MiB + 7, 4 * MiB,
+            for (size_t n : {(size_t)0, (size_t)1, MiB - 1, MiB, MiB + 1, 5 * MiB / 4, 2 * MiB - 1, 2 * MiB, 2 * MiB + 1, 5 * MiB / 2, 3 * MiB + 7, 4 * MiB,
                              4 * MiB + 1, 8 * MiB - 1, 8 * MiB, 8 * MiB + 1, 17 * MiB / 2, 12 * MiB, 12 * MiB + 5, 16 * MiB,
                              32 * MiB + 3, 70 * MiB + 1, 5 * MiB, (size_t)100})
                 both_ways(c, n, (uint32_t)n + 1u);
@@ -268,9 +269,11 @@ int main(int argc, char** argv)
         else if (what == "setup")
         {
             /* small copies make no staging; no copy makes more than 4 MiB */
-            for (size_t n : {(size_t)1, MiB, 2 * MiB - 1})
+            for (size_t n : {(size_t)1, MiB / 2, MiB - 1})
                 both_ways(c, n, 4u);
             expect(pinned_calls == 0, "pinned allocations of small copies", pinned_calls, 0);
+            both_ways(c, MiB + 1, 4u);
+            expect(pinned_total < 2 * MiB, "staging of 1 MiB", pinned_total, 2 * MiB);
             both_ways(c, 70 * MiB + 1, 4u);
             expect(pinned_total <= 4 * MiB, "staging", pinned_total, 4 * MiB);
         }
