@@ -9,12 +9,12 @@ import ctypes as C
 
 import numpy as np
 import pytest
-import torch
 
 import guide_ref as G
 from colvillea_amd import Integrator, IntegratorType, scenes, upload_scene
 from colvillea_amd import _capi as capi
 from colvillea_amd.integrator import View
+from test_zz_no_alloc import DeviceArray
 
 pytestmark = pytest.mark.gpu
 
@@ -43,13 +43,19 @@ def test_film_readback(size):
 def test_readback_into_pinned_memory():
     w, h = 512, 300  # 2.3 MiB
     desc = scenes.make_c0(width=w, height=h, spp=1, hdri_w=64, hdri_h=32)
-    out = torch.zeros((h, w, 4), dtype=torch.float32, pin_memory=True)
-    with Integrator.createIntegrator(IntegratorType.WavefrontPathTracing, w, h) as integ:
-        upload_scene(integ, desc)
-        integ.render(1)
-        capi.check(capi.lib().clhip_readback(integ.ctx, C.cast(out.data_ptr(), C.POINTER(C.c_float)), out.numel() * 4),
-                   integ.ctx)
-        assert np.array_equal(out.numpy(), integ.readbackFramebufferLinear())
+    hip = DeviceArray.hip()
+    own = C.c_void_p()
+    assert hip.hipHostMalloc(C.byref(own), C.c_size_t(16 * w * h), 0) == 0
+    try:
+        out = np.ctypeslib.as_array(C.cast(own, C.POINTER(C.c_float)), (h, w, 4))
+        out[:] = 7.0
+        with Integrator.createIntegrator(IntegratorType.WavefrontPathTracing, w, h) as integ:
+            upload_scene(integ, desc)
+            integ.render(1)
+            capi.check(capi.lib().clhip_readback(integ.ctx, C.cast(own, C.POINTER(C.c_float)), out.nbytes), integ.ctx)
+            assert np.array_equal(out, integ.readbackFramebufferLinear())
+    finally:
+        hip.hipHostFree(own)
 
 
 @pytest.mark.parametrize("n", [1, 20165, 20166, 40329, 40330, 60000, 80661, 700001])
