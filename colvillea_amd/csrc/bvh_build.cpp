@@ -4,8 +4,8 @@
  *
  * Binned SAH (32 bins per axis) produces a binary tree, which is collapsed
  * to a 4- or 8-wide tree by repeatedly opening the child with the largest
- * surface area.  BVH4 nodes are 128-byte Node4 records with float boxes
- * (eight 16-byte loads); BVH8 nodes are 96-byte Node8 records with child
+ * surface area.  BVH4 nodes are built as Node4 records with float boxes,
+ * which traversal reads packed to 80 bytes (Node4P); BVH8 nodes are 96-byte Node8 records with child
  * boxes quantised to bytes against the node's box, in the spirit of Ylitie,
  * Karras and Laine, "Efficient Incoherent Ray Traversal on GPUs Through
  * Compressed Wide BVHs", HPG 2017 (six 16-byte loads).

@@ -610,8 +610,10 @@ clpt::GuideTrainBufs guide_bufs(clhip_ctx* c)
 }
 
 /* A grid of about `blocks` blocks as the segmented queues need it: a
- * multiple of CLPT_SEGS, not above `blocks` (a persistent grid may not
- * exceed the resident blocks) unless that is none at all. */
+ * multiple of CLPT_SEGS, not above `blocks` (a persistent grid of more than
+ * the resident blocks ends with the late ones' shares) unless that is none at
+ * all.  The launch that closest-hit and any-hit rays share holds both grids,
+ * about twice what fits: see k_trace_shadow. */
 uint32_t seg_grid(uint32_t blocks) { return std::max(CLPT_SEGS, blocks / CLPT_SEGS * CLPT_SEGS); }
 
 /* Grid sizes from the launch shape (zero = default). */

@@ -25,11 +25,11 @@ namespace clpt
  * One HostCopier serves one context (it is not thread-safe).  Its staging and
  * threads are made at the first copy that needs them and kept for the
  * context's life; the host's first touch of new pinned memory costs 100 us
- * and more per MiB with all threads, so there is little of it.  Film of 1920x1080 (31.6 MiB) read back
- * after a render, first and later times in a context: 1.9 and 1.9 ms through
- * the runtime, 3.1 and 1.08 with 32 slots of 1 MiB each queued once, 0.89 and
- * 0.85 with these two; two slots of 1 MiB 1.07 later, of 4 MiB or four of 2
- * MiB no faster and up to 1 ms longer the first time.  Below kMin nothing is
+ * and more per MiB with all threads, so there is little of it.  A film of
+ * 1920x1080 (31.6 MiB) read back, first and later times in a context: 1.9 and
+ * 1.9 ms through the runtime, 3.1 and 1.08 with 32 slots of 1 MiB each queued
+ * once, 1.0 and 0.85 with these two; two slots of 1 MiB 1.07 later, of 4 MiB
+ * or four of 2 MiB no faster and up to 1 ms longer the first time.  Below kMin nothing is
  * gained (0.3 MiB takes 39 us, staged 45); behind a render 1.2 MiB staged is
  * 13 us sooner than the runtime's, which starts when the render has ended. */
 class HostCopier

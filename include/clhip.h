@@ -136,8 +136,10 @@ typedef struct
     uint64_t trace_tris;                   /* triangles tested by closest-hit traversal */
     uint64_t shadow_nodes;                 /* BVH4 nodes fetched by any-hit traversal */
     uint64_t shadow_tris;                  /* triangles tested by any-hit traversal */
-    uint64_t trace_launches;               /* closest-hit kernel launches */
-    uint64_t shadow_launches;              /* any-hit kernel launches */
+    uint64_t trace_launches;               /* closest-hit passes: one per depth and batch */
+    uint64_t shadow_launches;              /* any-hit passes: one per depth but the last.  A pass is a launch of
+                                              its own while timing is on; else a depth's any-hit pass and the
+                                              next depth's closest-hit pass are one launch */
     double   trace_ms;                     /* summed closest-hit kernel time (events; when timing is on) */
     double   shade_ms;                     /* summed shading kernel time */
     double   shadow_ms;                    /* summed any-hit kernel time */
@@ -172,8 +174,8 @@ int clhip_create_texture_u8(clhip_ctx* ctx, const uint8_t* data, uint32_t width,
 
 /* Tree width of the acceleration structures built from now on: 4 (default;
  * 80-byte nodes with half-float boxes) or 8 (96-byte nodes with child boxes
- * quantised to bytes); the stored boxes contain the exact ones.  No reference counterpart (OptiX builds its own).
- * Results do not depend on it; changing it requires building the BLAS and
+ * quantised to bytes); the stored boxes contain the exact ones.  No
+ * reference counterpart (OptiX builds its own).  Results do not depend on it; changing it requires building the BLAS and
  * TLAS again. */
 int clhip_set_bvh_width(clhip_ctx* ctx, uint32_t width);
 
@@ -248,7 +250,8 @@ int clhip_readback_sums(clhip_ctx* ctx, double* rgb, size_t bytes);
 
 /* Counters of the last render (queue counts, node/triangle fetches, kernel
  * times).  timing != 0 records HIP events around every traversal and
- * shading launch from the next render on. */
+ * shading launch from the next render on, for which closest-hit and any-hit
+ * rays are traced in launches of their own (the same results). */
 int clhip_counters(clhip_ctx* ctx, clhip_stats* out);
 int clhip_set_timing(clhip_ctx* ctx, int timing);
 
