@@ -451,6 +451,11 @@ def main():
                        "peak": L2_PEAK_GBS, "unit": "GB/s", "frac": round(req_gbs / L2_PEAK_GBS, 4),
                        "measured": meas.get("l2") if meas else None},
                 "limiter": meas.get("limiter") if meas else None,
+                # the times and counts above are from a render with event timing,
+                # which issues closest-hit and any-hit rays apart
+                "launches": "k_trace of each depth, any-hit rays apart (event timing); a render without it runs k_trace "
+                            "for the camera rays and shares k_trace_shadow between later rays and shadow rays",
+                "k_trace_shadow": meas.get("k_trace_shadow") if meas else None,
                 "counters_source": "profiles/k_trace_c1_1080p.md" if meas else None}
     import ctypes as C
 
