@@ -1171,7 +1171,7 @@ int clhip_create(uint32_t width, uint32_t height, uint32_t integrator_type, clhi
     c->cam.width  = width;
     c->cam.height = height;
     c->cam.npix   = width * height;
-    c->copier = std::make_unique<clpt::HostCopier>();
+    c->copier = std::make_unique<clpt::HostCopier>(c->device);
     *out         = c.release();
     return CLHIP_OK;
 }

@@ -48,7 +48,9 @@ void HostCopier::wait_upload(size_t k)
 
 bool HostCopier::reserve(size_t bytes)
 {
-    if (refused_)
+    /* events are the current device's, and the stream takes its own's only */
+    int device = -1;
+    if (refused_ || hipGetDevice(&device) != hipSuccess || device != device_)
         return false;
     for (size_t k = 0; k < kSlots; ++k)
         wait_upload(k);

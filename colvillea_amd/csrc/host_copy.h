@@ -35,7 +35,7 @@ namespace clpt
 class HostCopier
 {
 public:
-    HostCopier() = default;
+    explicit HostCopier(int device) : device_(device) {}
     ~HostCopier();
     HostCopier(const HostCopier&) = delete;
     HostCopier& operator=(const HostCopier&) = delete;
@@ -66,6 +66,7 @@ private:
     void finish();
     void work();
 
+    int                      device_; /* the streams' */
     char*                    stage_ = nullptr;
     size_t                   room_ = 0, slots_ = 0;
     bool                     touched_ = true;

@@ -24,6 +24,7 @@ size_t                            pinned_total = 0, pinned_calls = 0;
 size_t                            staged_copies = 0, direct_copies = 0;
 int                               waiting = 0; /* threads inside hipEventSynchronize */
 hipError_t                        last = hipSuccess;
+int                               current_device = 0; /* the stream's is 0 */
 
 bool in_pinned(const void* p)
 {
@@ -84,6 +85,7 @@ void expect(bool good, const char* what, size_t a, size_t b)
 struct ihipEvent_t
 {
     std::atomic<uint64_t> at{0};
+    int                   device = current_device;
 };
 
 extern "C" {
@@ -139,6 +141,8 @@ hipError_t hipEventDestroy(hipEvent_t e)
 }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t)
 {
+    if (e->device != 0)
+        return last = hipErrorInvalidHandle; /* not the stream's device */
     e->at = enqueue([] {});
     return hipSuccess;
 }
@@ -161,6 +165,11 @@ hipError_t hipStreamSynchronize(hipStream_t)
         at = queued;
     }
     wait_for(at);
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int* d)
+{
+    *d = current_device;
     return hipSuccess;
 }
 hipError_t hipGetLastError(void)
@@ -205,7 +214,7 @@ int main(int argc, char** argv)
     const std::string what = argc > 1 ? argv[1] : "";
     std::thread       dev(device);
     {
-        HostCopier c;
+        HostCopier c(0);
         if (what == "sizes")
         {
             /* around pieces, the sizes from which several threads copy, the
@@ -276,6 +285,17 @@ int main(int argc, char** argv)
             expect(pinned_total < 2 * MiB, "staging of 1 MiB", pinned_total, 2 * MiB);
             both_ways(c, 70 * MiB + 1, 4u);
             expect(pinned_total <= 4 * MiB, "staging", pinned_total, 4 * MiB);
+        }
+        else if (what == "device")
+        {
+            /* another device is current at the first large copy */
+            current_device = 1;
+            both_ways(c, 5 * MiB + 3, 6u);
+            expect(staged_copies == 0, "staged copies", staged_copies, 0);
+            current_device = 0;
+            both_ways(c, 5 * MiB + 3, 7u);
+            expect(staged_copies > 0, "staged copies", staged_copies, 1);
+            expect(hipGetLastError() == hipSuccess, "error left", 0, 0);
         }
         else
             expect(false, "unknown case", 0, 0);

@@ -26,7 +26,8 @@ def exe(tmp_path_factory):
 # pinned: the caller's own pinned memory takes one copy, not two
 # wait: behind a render still running only the calling thread waits
 # setup: small copies make no staging, large ones a bounded one
-@pytest.mark.parametrize("case", ["sizes", "no_pinned", "pinned", "wait", "setup"])
+# device: where another device than the context's is current, as it would be without staging
+@pytest.mark.parametrize("case", ["sizes", "no_pinned", "pinned", "wait", "setup", "device"])
 def test_copies(exe, case):
     r = subprocess.run([exe, case], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
