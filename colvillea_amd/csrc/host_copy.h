@@ -20,7 +20,7 @@ namespace clpt
  * pinned slots, and kThreads threads copy the parts out (or in) as they
  * arrive; a slot is queued again as soon as it is empty.  Copies below kMin,
  * copies to and from memory that is not pageable, and all copies where no
- * pinned memory can be had, go the runtime's way.
+ * pinned memory can be had or another device is current, go the runtime's way.
  *
  * One HostCopier serves one context (it is not thread-safe).  Its staging and
  * threads are made at the first copy that needs them and kept for the
