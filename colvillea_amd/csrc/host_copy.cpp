@@ -23,6 +23,8 @@ HostCopier::~HostCopier()
     }
     if (stage_)
         (void)hipHostFree(stage_);
+    if (tiny_)
+        (void)hipHostFree(tiny_);
 }
 
 /* Whether p is ordinary memory, which the runtime would copy through staging
@@ -173,11 +175,36 @@ void HostCopier::finish()
     idle_.wait(l, [&] { return busy_ == 0; });
 }
 
+bool HostCopier::tiny()
+{
+    if (!tiny_ && !refused_ && ++ntiny_ > 2u)
+    {
+        void* p = nullptr;
+        if (hipHostMalloc(&p, kTiny, hipHostMallocDefault) == hipSuccess)
+            tiny_ = p;
+        else
+        {
+            (void)hipGetLastError();
+            refused_ = true;
+        }
+    }
+    return tiny_ != nullptr;
+}
+
 hipError_t HostCopier::to_host(hipStream_t s, void* dst, const void* dev, size_t bytes)
 {
     if (!bytes)
         return hipStreamSynchronize(s);
     hipError_t e = hipSuccess;
+    if (bytes <= kTiny && tiny())
+    {
+        e = hipMemcpyAsync(tiny_, dev, bytes, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess)
+            e = hipStreamSynchronize(s);
+        if (e == hipSuccess)
+            std::memcpy(dst, tiny_, bytes);
+        return e;
+    }
     if (bytes < kMin || !pageable(dst) || !reserve(bytes))
     {
         e = hipMemcpyAsync(dst, dev, bytes, hipMemcpyDeviceToHost, s);

@@ -31,7 +31,10 @@ namespace clpt
  * once, 1.0 and 0.85 with these two; two slots of 1 MiB 1.07 later, of 4 MiB
  * or four of 2 MiB no faster and up to 1 ms longer the first time.  Below kMin nothing is
  * gained (0.3 MiB takes 39 us, staged 45); behind a render 1.2 MiB staged is
- * 13 us sooner than the runtime's, which starts when the render has ended. */
+ * 13 us sooner than the runtime's, which starts when the render has ended.
+ * But up to 16 KiB the runtime has a slower way to pageable memory: such
+ * readbacks go through a slot of that size from a context's third on (one
+ * alone would not repay it), 19.6 instead of 26 us each. */
 class HostCopier
 {
 public:
@@ -47,6 +50,7 @@ public:
     hipError_t from_host(hipStream_t s, void* dev, const void* src, size_t bytes);
 
 private:
+    static constexpr size_t   kTiny    = 16u << 10;
     static constexpr size_t   kMin     = 1u << 20;
     static constexpr size_t   kPart    = 2u << 20; /* one transfer, one slot */
     static constexpr size_t   kSlots   = 2;
@@ -57,6 +61,8 @@ private:
     /* staging and events for a copy; false: there are none to be had */
     bool reserve(size_t bytes);
     void touch();
+    /* the slot of tiny readbacks, once there have been several */
+    bool tiny();
     void wait_upload(size_t k);
     /* job(k) for k = 0..n-1 on the threads from begin() on; the caller's takes
      * those below `end` that are left in help() and all in finish(), which
@@ -68,6 +74,8 @@ private:
 
     int                      device_; /* the streams' */
     char*                    stage_ = nullptr;
+    void*                    tiny_  = nullptr;
+    unsigned                 ntiny_ = 0;
     size_t                   room_ = 0, slots_ = 0;
     bool                     touched_ = true;
     bool                     refused_ = false; /* pinned memory or an event could not be had */

@@ -221,7 +221,7 @@ int main(int argc, char** argv)
              * whole staging and several times it, up and down in turn */
             for (size_t n : {(size_t)0, (size_t)1, MiB - 1, MiB, MiB + 1, 5 * MiB / 4, 2 * MiB - 1, 2 * MiB, 2 * MiB + 1, 5 * MiB / 2, 3 * MiB + 7, 4 * MiB,
                              4 * MiB + 1, 8 * MiB - 1, 8 * MiB, 8 * MiB + 1, 17 * MiB / 2, 12 * MiB, 12 * MiB + 5, 16 * MiB,
-                             32 * MiB + 3, 70 * MiB + 1, 5 * MiB, (size_t)100})
+                             32 * MiB + 3, 70 * MiB + 1, 5 * MiB, (size_t)100, (size_t)16383, (size_t)16384, (size_t)16385, (size_t)3})
                 both_ways(c, n, (uint32_t)n + 1u);
         }
         else if (what == "no_pinned")
@@ -229,7 +229,7 @@ int main(int argc, char** argv)
             /* no pinned memory: the copies go the runtime's way, and leave no
              * error for the next launch to report */
             refuse_pinned = true;
-            for (size_t n : {(size_t)100, 3 * MiB, 40 * MiB + 1})
+            for (size_t n : {(size_t)100, 3 * MiB, 40 * MiB + 1, (size_t)7, (size_t)8, (size_t)9})
                 both_ways(c, n, 3u);
             expect(hipGetLastError() == hipSuccess, "error left", 0, 0);
             expect(staged_copies == 0, "staged copies", staged_copies, 0);
@@ -281,10 +281,18 @@ int main(int argc, char** argv)
             for (size_t n : {(size_t)1, MiB / 2, MiB - 1})
                 both_ways(c, n, 4u);
             expect(pinned_calls == 0, "pinned allocations of small copies", pinned_calls, 0);
+            for (uint32_t k = 0; k < 5u; ++k)
+            {
+                both_ways(c, 16384u, k);
+                both_ways(c, 1u + 100u * k, k);
+            }
+            expect(pinned_calls == 1 && pinned_total == 16384u, "pinned memory of tiny copies", pinned_calls, pinned_total);
+            both_ways(c, 16385u, 4u);
+            expect(pinned_calls == 1, "pinned allocations of small copies", pinned_calls, 1);
             both_ways(c, MiB + 1, 4u);
             expect(pinned_total < 2 * MiB, "staging of 1 MiB", pinned_total, 2 * MiB);
             both_ways(c, 70 * MiB + 1, 4u);
-            expect(pinned_total <= 4 * MiB, "staging", pinned_total, 4 * MiB);
+            expect(pinned_total <= 4 * MiB + 16384u, "staging", pinned_total, 4 * MiB);
         }
         else if (what == "device")
         {

@@ -25,7 +25,7 @@ def exe(tmp_path_factory):
 # no_pinned: without pinned memory copies still work
 # pinned: the caller's own pinned memory takes one copy, not two
 # wait: behind a render still running only the calling thread waits
-# setup: small copies make no staging, large ones a bounded one
+# setup: tiny readbacks make 16 KiB of pinned memory, once there are several; small copies none, large ones a bounded staging
 # device: where another device than the context's is current, as it would be without staging
 @pytest.mark.parametrize("case", ["sizes", "no_pinned", "pinned", "wait", "setup", "device"])
 def test_copies(exe, case):
