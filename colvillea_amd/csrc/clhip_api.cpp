@@ -2241,9 +2241,8 @@ int clhip_counters(clhip_ctx* ctx, clhip_stats* out)
             const WaveCounts wc{ctx->d_ctr.as<unsigned long long>(), ctx->wc_stride};
             CLHIP_CHECK(ctx, clpt::launch_sum_waves(ctx->stream, wc, wc_rows(ctx->wc_depth),
                                                     ctx->d_tot.as<TotalCounters>()));
-            CLHIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
         }
-        CLHIP_CHECK(ctx, hipMemcpy(&t, ctx->d_tot.p, sizeof(t), hipMemcpyDeviceToHost));
+        CLHIP_CHECK(ctx, ctx->copier->to_host(ctx->stream, &t, ctx->d_tot.p, sizeof(t)));
         for (int b = 0; b <= CLHIP_MAX_DEPTH && b < CLPT_MAXD + 2; ++b)
         {
             out->rays[b]    = t.rays[b];

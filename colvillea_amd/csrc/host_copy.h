@@ -29,12 +29,12 @@ namespace clpt
  * 1920x1080 (31.6 MiB) read back, first and later times in a context: 1.9 and
  * 1.9 ms through the runtime, 3.1 and 1.08 with 32 slots of 1 MiB each queued
  * once, 1.0 and 0.85 with these two; two slots of 1 MiB 1.07 later, of 4 MiB
- * or four of 2 MiB no faster and up to 1 ms longer the first time.  Below kMin nothing is
- * gained (0.3 MiB takes 39 us, staged 45); behind a render 1.2 MiB staged is
- * 13 us sooner than the runtime's, which starts when the render has ended.
- * But up to 16 KiB the runtime has a slower way to pageable memory: such
- * readbacks go through a slot of that size from a context's third on (one
- * alone would not repay it), 19.6 instead of 26 us each. */
+ * or four of 2 MiB no faster and up to 1 ms longer the first time.  Below
+ * kMin nothing is gained (0.3 MiB takes 39 us, staged 45); behind a render
+ * 1.2 MiB staged is 13 us sooner than the runtime's, which starts when the
+ * render has ended.  But up to 16 KiB the runtime has a slower way to
+ * pageable memory: such readbacks go through a slot of that size from a
+ * context's third on (one alone would not repay it), 18 instead of 26 us. */
 class HostCopier
 {
 public:
